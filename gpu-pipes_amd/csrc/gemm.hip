@@ -44,18 +44,11 @@
 #include <utility>
 
 #include "../../include/gpipes.h"
-#include "gp_device.hpp"
-#include "gp_kernels.hpp"
-#include "stages.hpp"
+#include "gemm_common.hpp"
 
 namespace gp {
 namespace gemm {
 
-constexpr int BK = 64;              // k per slab
-constexpr int ROWB = BK * 2;        // bytes per unit row (one 128-byte L2 line)
-constexpr int CPR = ROWB / 16;      // 16-byte chunks per row
-constexpr int RPC = 1024 / ROWB;    // rows per 1 KiB copy instruction
-constexpr int KS = BK / 16;         // MFMA k-steps per slab
 constexpr int NU = 5;               // units in the LDS ring
 constexpr int NW = 4;               // waves per workgroup
 constexpr int kLnPasses = 4;        // passes over the grid one LayerNorm-exchange launch may run
@@ -78,38 +71,6 @@ using Narrow = Cfg<4, 2, 1>;  // 128 features x 256 rows
 using Short = Cfg<4, 1, 1>;   // 128 features x 128 rows: N = 128 LayerNorm launches of fewer rows than 256 per CU
 
 // Element types: F16 / BF16 (gp_device.hpp).
-
-
-struct Args {
-  const half_t* a;     // [M][lda], the first K columns used
-  const half_t* bt;    // [N][K] (transposed weights), or
-  const half_t* w;     // [kw][ldw] (the weights in their own layout, BROW kernels)
-  int ldw, kw;         // row stride and rows of w; rows [kw, K) read as zero
-  const half_t* bias;  // [N] or null
-  const half_t* r;     // [M][ldr] residual or null
-  half_t* c;           // [M][ldc], the first N columns written
-  int64_t M;
-  int N;
-  int K;
-  int ka;              // columns of A read (a multiple of 8, <= K); columns [ka, K) read as zero
-  int lda, ldc, ldr;   // row strides in elements
-  // LayerNorm epilogue (LNM kernels): gamma / beta [N] or null (1 / 0), eps.
-  const half_t* gamma;
-  const half_t* beta;
-  float eps;
-  // LNM 2: per-row partial statistics [M][N / 128] ((mean, M2) of one wave's
-  // 128 features, as 64-bit words), per-row-block commit counters, and the
-  // launch context (epoch, status word, poll bound).
-  unsigned long long* stats;
-  QCounter* cnt;
-  QueueCtx ctx;
-  uint32_t ln_target;  // count of a row block's counter once this launch's waves have all committed
-};
-
-// Byte offset of logical 16-byte chunk c of unit row r: the chunk position is
-// XOR-swizzled with (r / 2) so 16 consecutive rows (two per 256-byte bank
-// window) read at one logical chunk cover 16 distinct 16-byte bank groups.
-__device__ __forceinline__ int unit_off(int r, int c) { return r * ROWB + ((c ^ ((r >> 1) & 7)) << 4); }
 
 template <typename F, int... I>
 __device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&& f) {
@@ -268,8 +229,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 #pragma unroll
       for (int nb = 0; nb < C::NBW; ++nb) {
         const int lb = lb0 ^ (64 * nb);
-        const s4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GP_LDS s4*)(ub + lb));
-        const s4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GP_LDS s4*)(ub + lb + 4 * (C::BN * 2)));
+        const s4 x0 = lds_tr16(ub + lb);
+        const s4 x1 = lds_tr16(ub + lb + 4 * (C::BN * 2));
         f.a[nb] = __builtin_bit_cast(h8, __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
       }
     } else {
@@ -696,8 +657,7 @@ __device__ __forceinline__ void transpose_tile64(const half_t* w, int K, int N, 
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
       const int r = 8 * kg + 4 * hh + (m >> 2), col = 16 * nb + 4 * (m & 3);
-      part[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (GP_LDS s4*)(tile + r * 128 + (((col >> 3) ^ (r & 7)) << 4) + (col & 7) * 2));
+      part[hh] = lds_tr16(tile + r * 128 + (((col >> 3) ^ (r & 7)) << 4) + (col & 7) * 2);
     }
     *(h8*)(wt + (int64_t)(n0 + 16 * nb + m) * Kp + k0 + 8 * kg) =
         __builtin_bit_cast(h8, __builtin_shufflevector(part[0], part[1], 0, 1, 2, 3, 4, 5, 6, 7));

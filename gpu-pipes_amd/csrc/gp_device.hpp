@@ -217,9 +217,19 @@ __device__ __forceinline__ int wrow_voff(int lane, int stride) {
 // four different chunk groups, so the read is conflict free.
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef short s8 __attribute__((ext_vector_type(8)));
+// The restrict qualifier gives the read an alias scope.  Without one the
+// compiler takes a transposing read for a possible reader of every
+// global->LDS copy in flight and waits for all of them (vmcnt(0)) before it;
+// callers wait for the copies they read themselves (wait_vmcnt).  The wide
+// GEMM with its weights in place, one K-slab ring drained per 16-k step before:
+// bert_ffn 509 x 1024 x 4096 180 -> 134 us a call, the DLRM MLPs at 2,048 rows
+// 137 -> 118 us, outputs bit-identical.
+__device__ __forceinline__ s4 lds_tr16(GP_LDS const char* __restrict p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((GP_LDS s4*)p);
+}
 __device__ __forceinline__ s4 wrows_col4(const GP_LDS char* blk, int fb, int m) {
   const int r = m >> 2, f = fb + 4 * (m & 3);
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((GP_LDS s4*)(blk + r * 256 + (((f >> 3) ^ (4 * r)) * 16) + (f & 7) * 2));
+  return lds_tr16(blk + r * 256 + (((f >> 3) ^ (4 * r)) * 16) + (f & 7) * 2);
 }
 // Eight consecutive k: lane j receives W[kb + e][fb + j], e = 0..7, from the
 // four-row blocks at blk0 (rows kb..kb+3) and blk1 (rows kb+4..kb+7).
