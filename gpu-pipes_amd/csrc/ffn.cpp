@@ -74,8 +74,16 @@ struct LnEpilogue {
   uint32_t epoch = 0;
   int64_t round = 0;
 
-  int init(int dev, hipStream_t s, int64_t rows, int64_t H) {
+  // exchange: some launch of the call runs its LayerNorm in the epilogue.
+  // Without one the call only registers itself (a clean status word), so that
+  // gp_pipeline_check answers for it as for any other.
+  int init(int dev, hipStream_t s, int64_t rows, int64_t H, bool exchange) {
     if (H == 128) return GP_OK;
+    if (!exchange) {
+      unsigned long long* word = nullptr;
+      uint32_t e = 0;
+      return status_acquire(dev, s, &word, &e);
+    }
     const int rc = arena_acquire(dev, s, gemm_ln_ws_bytes(rows, H), kArenaLayoutGemmLn, &ws, &epoch);
     if (rc) return rc;
     status_note(dev, s, (unsigned long long*)ws, epoch);
@@ -94,6 +102,15 @@ struct LnEpilogue {
       g.ln_round = round++;
     }
     return g;
+  }
+  // g (a GEMM with bias and residual) and the LayerNorm over its rows: one
+  // launch with the LayerNorm in the epilogue, or (also for a last short chunk
+  // of a call that took no exchange area) the GEMM's rows written to g.out and
+  // normalised there.
+  hipError_t launch(const GemmArgs& g, const void* gamma, const void* beta, float eps, int ncu, hipStream_t s) {
+    if (g.N == 128 || (ws && !gemm_ln_apart(g.M, g.N, g.K, ncu))) return gemm_launch(apply(g, gamma, beta, eps), ncu, s);
+    const hipError_t e = gemm_launch(g, ncu, s);
+    return e == hipSuccess ? gemm_ln_rows_launch(g.M, g.N, g.out, gamma, beta, eps, g.out, g.dtype, s) : e;
   }
 };
 
@@ -210,7 +227,7 @@ int gp_bert_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* x, const
     return ga;
   };
   LnEpilogue lne;
-  if (fuse_ln && (rc = lne.init(dev, s, CH, H))) return rc;
+  if (fuse_ln && (rc = lne.init(dev, s, CH, H, !gemm_ln_apart(CH, H, FF, ncu)))) return rc;
   for (int64_t r0 = 0; r0 < M; r0 += CH) {
     const int64_t rows = M - r0 < CH ? M - r0 : CH;
     const void* xc = at_row(x, r0, H);
@@ -218,8 +235,8 @@ int gp_bert_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* x, const
     e = gemm_launch(g(rows, FF, H, xc, w1, w1t, b1, nullptr, act, hbuf), ncu, s);
     if (e != hipSuccess) return fail_hip(e, "FFN GEMM1 launch");
     if (fuse_ln) {
-      // GEMM2 + bias + residual + LayerNorm in one launch
-      e = gemm_launch(lne.apply(g(rows, H, FF, hbuf, w2, w2t, b2, xc, GP_ACT_NONE, oc), gamma, beta, eps), ncu, s);
+      // GEMM2 + bias + residual + LayerNorm
+      e = lne.launch(g(rows, H, FF, hbuf, w2, w2t, b2, xc, GP_ACT_NONE, oc), gamma, beta, eps, ncu, s);
       if (e != hipSuccess) return fail_hip(e, "FFN GEMM2 + LayerNorm launch");
       continue;
     }
@@ -333,17 +350,17 @@ int gp_bert_addln_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* at
     return ga;
   };
   LnEpilogue lne;
-  if (fuse_ln && (rc = lne.init(dev, s, CH, H))) return rc;
+  if (fuse_ln && (rc = lne.init(dev, s, CH, H, !gemm_ln_apart(CH, H, H, ncu) || !gemm_ln_apart(CH, H, FF, ncu)))) return rc;
   for (int64_t r0 = 0; r0 < M; r0 += CH) {
     const int64_t rows = M - r0 < CH ? M - r0 : CH;
     if (fuse_ln) {
       // GEMM0 + b0 + x + LN0, GEMM1 + b1 + act, GEMM2 + b2 + h0 + LN2
       char* const oc = (char*)out + r0 * H * 2;
-      e = gemm_launch(lne.apply(g(rows, H, H, at_row(attn, r0, H), w0, w0t, b0, at_row(x, r0, H), GP_ACT_NONE, h0),
-                                ga0, be0, eps), ncu, s);
+      e = lne.launch(g(rows, H, H, at_row(attn, r0, H), w0, w0t, b0, at_row(x, r0, H), GP_ACT_NONE, h0), ga0, be0, eps,
+                     ncu, s);
       if (e == hipSuccess) e = gemm_launch(g(rows, FF, H, h0, w1, w1t, b1, nullptr, act, abuf), ncu, s);
       if (e == hipSuccess)
-        e = gemm_launch(lne.apply(g(rows, H, FF, abuf, w2, w2t, b2, h0, GP_ACT_NONE, oc), ga2, be2, eps), ncu, s);
+        e = lne.launch(g(rows, H, FF, abuf, w2, w2t, b2, h0, GP_ACT_NONE, oc), ga2, be2, eps, ncu, s);
       if (e != hipSuccess) return fail_hip(e, "bert_addln_ffn launch");
       continue;
     }

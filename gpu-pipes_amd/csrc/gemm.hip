@@ -40,6 +40,7 @@
 //    the tile's valid rows, so partial tiles need no per-row branches.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -765,6 +766,33 @@ static hipError_t launch_typed(const GemmArgs& a, Args& g, bool brow, int num_cu
   return brow ? dispatch<Narrow, true, E>(g, a.act, num_cus, s) : dispatch<Narrow, false, E>(g, a.act, num_cus, s);
 }
 
+// Time of one launch in microseconds, by the tile it runs on: a start, then
+// per round of tiles over the CUs a K walk (microseconds per 64-k slab, more
+// when every CU copies at once) and an epilogue.  Fitted to 23 shapes, M 64 ..
+// 65,536, N 128 .. 4096, K 128 .. 4096 (fp16, weights in place, one kernel at
+// a time); within 15% of nearly all and with the fastest kernel of the three
+// on every one of them, e.g. 256-row / 128 x 128 / 64 x 64 tiles:
+//   509 x 1024 x 4096    82 / 34 / 16 us     2048 x 1024 x 1024   26 / 13 / 10
+//   4096 x 1024 x 4096   89 / 41 / 66        8192 x 1024 x 4096   94 / 79 / 141
+//   4096 x 4096 x 1024   38 / 59 / 84        16384 x 1024 x 1024  37 / 50 / 56
+struct TileCost {
+  double best;
+  int size;  // 0: the persistent 256-row kernels; 64, 128: gemm_tile.hip
+};
+static TileCost tile_cost(int64_t M, int64_t N, int64_t K, int num_cus) {
+  const double slabs = (double)(K / BK);
+  auto tiles = [&](int64_t bm, int64_t bn) { return (double)((M + bm - 1) / bm) * (double)(N / bn); };
+  auto rounds = [&](double t, int per_cu) { return ceil(t / (num_cus * per_cu)); };
+  auto load = [&](double t) { return t < num_cus ? t / num_cus : 1.0; };
+  const bool wide = N % Wide::BN == 0;
+  const double t256 = tiles(256, wide ? 256 : 128), t128 = tiles(128, 128), t64 = tiles(64, 64);
+  const double c256 = 5.0 + rounds(t256, 1) * (slabs * (wide ? 1.0 : 0.55) * (1.15 + 0.75 * load(t256)) + 3.0);
+  const double c128 = 2.5 + rounds(t128, 1) * (slabs * (0.45 + 0.12 * load(t128)) + 3.0);
+  const double c64 = 3.0 + rounds(t64, 2) * (slabs * (t64 > num_cus ? 0.42 : 0.21) + 1.2);
+  if (c256 <= c128 && c256 <= c64) return {c256, 0};
+  return c128 <= c64 ? TileCost{c128, 128} : TileCost{c64, 64};
+}
+
 // The LNM 2 exchange area: the status word's line, kLnMaxBlocks counter
 // lines (one per row block of a launch: a Wide tile row), then 8 bytes per
 // row and wave of partial statistics.  The counters sit at the same place whatever the
@@ -823,7 +851,21 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t s) {
       g.ln_target = (uint32_t)((a.ln_round + 1) * tiles_n * NW);
     }
   }
+  if (!a.ln)
+    if (const int size = tile_cost(a.M, a.N, a.K, num_cus).size) return tile_launch(g, a.act, size, a.dtype, s);
   return a.dtype == GP_DTYPE_BF16 ? launch_typed<BF16>(a, g, brow, num_cus, s) : launch_typed<F16>(a, g, brow, num_cus, s);
+}
+
+bool gemm_ln_apart(int64_t M, int64_t N, int64_t K, int num_cus) {
+  using namespace gemm;
+  if (N == 128 || M <= 0) return false;
+  const TileCost c = tile_cost(M, N, K, num_cus);
+  if (c.size == 0) return false;
+  // The epilogue rides on the 256-row kernel and adds the statistics exchange
+  // (about 4 us); a launch of its own costs about 3.5 us and 4 bytes an element.
+  const double slabs = (double)(K / BK), t = (double)((M + 255) / 256) * (double)(N / 256);
+  const double fused = 5.0 + slabs * (1.15 + 0.75 * (t < num_cus ? t / num_cus : 1.0)) + 7.0;
+  return c.best + 3.5 + 4e-6 * (double)M * (double)N / 4.0 < fused;
 }
 
 hipError_t prep_launch(const PrepSpec* L, int n, hipStream_t s) {

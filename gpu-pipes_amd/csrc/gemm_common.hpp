@@ -45,6 +45,10 @@ struct Args {
   uint32_t ln_target;  // count of a row block's counter once this launch's waves have all committed
 };
 
+// Small-tile kernels (gemm_tile.hip): one `size` x `size` output tile per
+// workgroup (64 or 128); p.bt or p.w as in gemm_launch, no LayerNorm epilogue.
+hipError_t tile_launch(const Args& p, int act, int size, int dtype, hipStream_t s);
+
 // Byte offset of logical 16-byte chunk c of unit row r: the chunk position is
 // XOR-swizzled with (r / 2) so 16 consecutive rows (two per 256-byte bank
 // window) read at one logical chunk cover 16 distinct 16-byte bank groups.

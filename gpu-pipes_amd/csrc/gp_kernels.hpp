@@ -153,6 +153,16 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t stream);
 // size of its exchange area.
 int64_t gemm_ln_max_rows(int64_t N, int num_cus);
 size_t gemm_ln_ws_bytes(int64_t M, int64_t N);
+// Whether a GEMM that ends in a LayerNorm runs faster as a small-tile GEMM
+// (its rows written out) and gemm_ln_rows_launch over them than with the
+// LayerNorm in its epilogue: few rows, which the epilogue's 256-row tiles
+// would spread over few CUs.  The two give the same bits.
+bool gemm_ln_apart(int64_t M, int64_t N, int64_t K, int num_cus);
+// out = LayerNorm(x) over rows of N (128, 256, 512 or 1024) finished 16-bit
+// values, with the statistics of the GEMM's LayerNorm epilogue bit for bit;
+// gamma / beta may be null (1 / 0).  In place when out == x.
+hipError_t gemm_ln_rows_launch(int64_t M, int64_t N, const void* x, const void* gamma, const void* beta, float eps,
+                               void* out, int dtype, hipStream_t s);
 // Whether a layer chain reads its weights in place instead of from
 // transposed copies.  In place, each weight fragment of the GEMM's k-loop
 // takes two transposing LDS reads instead of one 16-byte read, which slows

@@ -327,3 +327,51 @@ def test_bert_ffn_pipelined_refuses_capture(cuda):
     gpipes.bert_ffn_out(*args[:-1], out2, impl="pipelined")
     gpipes.pipeline_check()
     assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
+
+
+# ------------------------------------------------------------------ small tiles
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,K,act,resid", [(128, 64, "relu", False), (384, 320, "gelu_tanh", False),
+                                           (1024, 192, "none", True), (256, 1088, "sigmoid", False)])
+def test_gemm_tile_sizes_agree(cuda, N, K, act, resid, dtype):
+    """Few rows run on 64 x 64 or 128 x 128 tiles, many on 256-row ones; every
+    row's products are added in one order, so a call of any number of rows gives
+    the bits of the same rows in the largest call.  Row counts around the tile
+    edges; K from one slab to more slabs than the ring holds."""
+    M = 70001 if N <= 384 else 20001
+    x = normal_fp16(M, K, seed=N, device=cuda, dtype=dtype)
+    w = (normal_fp16(K, N, seed=K, device=cuda).float() / K ** 0.5).to(dtype)
+    b = normal_fp16(1, N, seed=3, device=cuda, dtype=dtype)[0]
+    r = normal_fp16(M, N, seed=4, device=cuda, dtype=dtype) if resid else None
+    big = gpipes.gemm_out(x, w, b, r, act=act)
+    rows = np.r_[0:64, M - 64:M]
+    got, xs = f(big[rows]), f(x[rows])
+    want = oracle.linear(xs, f(w), f(b), ACT_ID[act]) + (f(r[rows]) if resid else 0)
+    # 16-bit rounding of the result: 2^-11 (fp16) or 2^-8 (bf16) of a value, under 2^-10 / 2^-7 in the 2-norm
+    assert np.linalg.norm(got - want) <= (2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7) * np.linalg.norm(want)
+    for n in (1, 63, 64, 65, 127, 129, 255, 300, 1000, 4097, 9000):
+        small = gpipes.gemm_out(x[:n], w, b, None if r is None else r[:n], act=act)
+        assert torch.equal(small.view(torch.int16), big[:n].view(torch.int16)), (n, N, K)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H,FF", [(256, 1024), (512, 384), (1024, 2048)])
+def test_bert_ffn_small_batches_match_large(cuda, H, FF, dtype):
+    """Few rows run the LayerNorm as a launch over GEMM2's rows, many in GEMM2's
+    epilogue with the exchange between workgroups: the same statistics in the
+    same order, so the same bits; with and without the affine, in place too."""
+    M = 66000
+    p = {k: v.to(dtype) for k, v in dev(bert_params(H, FF, seed=H, init="bert", affine_random=True), cuda).items()}
+    x = normal_fp16(M, H, seed=1, device=cuda, dtype=dtype)
+    for ga, be in ((p["gamma"], p["beta"]), (None, None)):
+        def call(v, out):
+            return gpipes.bert_ffn_out(v, p["w1"], p["b1"], p["w2"], p["b2"], ga, be, out, eps=1e-12, act="gelu_tanh")
+        big = call(x, torch.empty_like(x))
+        gpipes.pipeline_check()
+        for n in (1, 65, 500, 1031, 5000):
+            small = call(x[:n], torch.empty_like(x[:n]))
+            gpipes.pipeline_check()
+            assert torch.equal(small.view(torch.int16), big[:n].view(torch.int16)), n
+    v = x[:777].clone()
+    call(v, v)
+    assert torch.equal(v.view(torch.int16), big[:777].view(torch.int16))
