@@ -48,6 +48,7 @@
 #include "gp_device.hpp"
 #include "gp_host.hpp"
 #include "gp_kernels.hpp"
+#include "rows_split.hpp"
 #include "stages.hpp"
 
 namespace gp {
@@ -104,32 +105,7 @@ __device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&&
   (f(std::integral_constant<int, I>{}), ...);
 }
 
-// fp16 (bf16) pair of an accumulator block with an optional ReLU: lo holds
-// elements 0-7, hi 8-15.  In bf16 the ReLU is a signed 16-bit integer max on
-// the rounded bits (a bf16 value with its sign bit set becomes +0).
-template <typename E>
-__device__ __forceinline__ void to_operands(const f16x& a, bool relu, h8& lo, h8& hi) {
-  if constexpr (std::is_same_v<E, F16>) {
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      lo[r] = (half_t)a[r];
-      hi[r] = (half_t)a[8 + r];
-    }
-    if (relu) {
-      lo = __builtin_elementwise_max(lo, h8{});
-      hi = __builtin_elementwise_max(hi, h8{});
-    }
-  } else {
-    lo = __builtin_shufflevector(E::cvt4(f4{a[0], a[1], a[2], a[3]}), E::cvt4(f4{a[4], a[5], a[6], a[7]}), 0, 1, 2, 3,
-                                 4, 5, 6, 7);
-    hi = __builtin_shufflevector(E::cvt4(f4{a[8], a[9], a[10], a[11]}), E::cvt4(f4{a[12], a[13], a[14], a[15]}), 0, 1,
-                                 2, 3, 4, 5, 6, 7);
-    if (relu) {
-      lo = __builtin_bit_cast(h8, __builtin_elementwise_max(__builtin_bit_cast(s8, lo), s8{}));
-      hi = __builtin_bit_cast(h8, __builtin_elementwise_max(__builtin_bit_cast(s8, hi), s8{}));
-    }
-  }
-}
+using rows_split::to_operands;
 
 // E: F16 or BF16.  NKB1: k-blocks of the first layer (K0 <= 16 NKB1).
 template <typename E, int NKB1>

@@ -56,6 +56,7 @@
 #include "gp_device.hpp"
 #include "gp_host.hpp"
 #include "gp_kernels.hpp"
+#include "rows_split.hpp"
 #include "stages.hpp"
 
 namespace gp {
@@ -331,27 +332,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
           h8 lo, hi;
-          if constexpr (std::is_same_v<E, F16>) {
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-              lo[r] = (half_t)acc[fb][rb][r];
-              hi[r] = (half_t)acc[fb][rb][8 + r];
-            }
-            if (relu) {
-              lo = __builtin_elementwise_max(lo, h8{});
-              hi = __builtin_elementwise_max(hi, h8{});
-            }
-          } else {
-            const f16x& a = acc[fb][rb];
-            lo = __builtin_shufflevector(E::cvt4(f4{a[0], a[1], a[2], a[3]}), E::cvt4(f4{a[4], a[5], a[6], a[7]}), 0, 1,
-                                         2, 3, 4, 5, 6, 7);
-            hi = __builtin_shufflevector(E::cvt4(f4{a[8], a[9], a[10], a[11]}), E::cvt4(f4{a[12], a[13], a[14], a[15]}),
-                                         0, 1, 2, 3, 4, 5, 6, 7);
-            if (relu) {
-              lo = __builtin_bit_cast(h8, __builtin_elementwise_max(__builtin_bit_cast(s8, lo), s8{}));
-              hi = __builtin_bit_cast(h8, __builtin_elementwise_max(__builtin_bit_cast(s8, hi), s8{}));
-            }
-          }
+          rows_split::to_operands<E>(acc[fb][rb], relu, lo, hi);
           act[2 * fb][rb] = lo;
           act[2 * fb + 1][rb] = hi;
         }
@@ -549,6 +530,254 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   wait_vmcnt<0>();
 }
 
+// ------------------------------------------------------------- few rows
+// The same chain with the features split over the waves and 64 rows per
+// workgroup (rows_split.hpp), from the same packed weight stream.
+//
+// Weight fragments that every wave reads one of, in the order a wave consumes
+// them: layers 1-8 and 10 (eight feature blocks: wave w reads block w), then
+// layer 11 (four blocks: block w % 4; its k-blocks 2 and 3, past the 32 columns
+// of d, are zero and left out).  The heads (layers 9 and 12) are loaded by the
+// waves that compute them.
+namespace split {
+using namespace rows_split;
+constexpr int RB = rows_split::RB;  // (not the 256-row kernel's)
+
+struct Seg {
+  int n, slot, fb;
+};
+constexpr Seg kSeg[] = {{4, S_L1, 8},       {16, S_L2, 8},      {16, S_L2 + 8, 8}, {16, S_L2 + 16, 8},
+                        {16, S_L2 + 24, 8}, {20, S_L6, 8},      {16, S_L7, 8},     {16, S_L7 + 8, 8},
+                        {16, S_L10, 8},     {18, S_L11, 4}};
+constexpr int kTrunkFrags = 120, kAllFrags = 154, kFour = 136;  // fragments; the first of layer 11
+// Byte offset in the stream of fragment j, feature block 0.
+constexpr int seq_off(int j) {
+  int i = 0;
+  while (j >= kSeg[i].n) j -= kSeg[i++].n;
+  const int kb = kSeg[i].fb == 4 && j >= 2 ? j + 2 : j;
+  return kSeg[i].slot * SLOT + kb * kSeg[i].fb * FRAG;
+}
+
+constexpr int IMG = 16 * RB * FRAG;  // one 256-wide activation image
+constexpr int L_IMG = 0, L_XI = 2 * IMG, L_DI = L_XI + 4 * RB * FRAG, LDS_SPLIT = L_DI + 2 * RB * FRAG;
+
+template <typename E, bool TRUNK>
+__global__ __launch_bounds__(rows_split::NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void nerf_split_kernel(Args p) {
+  constexpr int T = TRUNK ? kTrunkFrags : kAllFrags;
+  constexpr int PF = TRUNK ? 15 : 14;  // fragments in flight per wave
+  static_assert(T % PF == 0, "a tile's first fragment takes register set 0");
+  constexpr int LB = 3;  // B operands are read from LDS this many k-blocks ahead
+  constexpr int TR = rows_split::ROWS;
+  __shared__ __attribute__((aligned(1024))) char smem[LDS_SPLIT];
+  GP_LDS char* const lds = (GP_LDS char*)smem;
+  const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  GP_LDS char* const mine = lds + 16 * lane;  // this lane's 16 bytes of fragment 0
+  const int ntiles = (int)((p.M + TR - 1) / TR);
+
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.stream, (TRUNK ? S_L9 : S_TOTAL) * SLOT);
+  const __amdgpu_buffer_rsrc_t rbias = make_rsrc(p.bias, B_TOTAL * 2);
+  const int v8 = 16 * lane + wave * FRAG, v4 = 16 * lane + (wave & 3) * FRAG;
+  h8 wf[PF];  // fragment j in register set j % PF
+  auto fetch = [&](auto jc, __amdgpu_buffer_rsrc_t r) {
+    constexpr int j = decltype(jc)::value;
+    constexpr int off = seq_off(j);
+    wf[j % PF] = load_frag(r, j >= kFour ? v4 : v8, off);
+  };
+  // Bias column of feature block fb (its A operand has the bias at k = 0).
+  auto bias_at = [&](int off, int fb) {
+    return (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rbias, (off + 64 * fb + lane) * 2, 0, 0);
+  };
+  h8 ones = {};
+  ones[0] = __builtin_bit_cast(half_t, lane < 32 ? E::kOne : (unsigned short)0);
+  auto biased = [&](unsigned short b) {
+    h8 a = {};
+    a[0] = __builtin_bit_cast(half_t, b);
+    return E::mma(a, ones, f16x{});
+  };
+
+  unsigned short bnext = bias_at(BF_L1, wave);
+  static_for(std::make_integer_sequence<int, PF>{}, [&](auto j) { fetch(j, rw); });
+
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const int64_t r0 = (int64_t)t * TR;
+    const int vrows = p.M - r0 < TR ? (int)(p.M - r0) : TR;
+    // Past the last tile the next tile's fragments come through an empty
+    // descriptor.
+    const __amdgpu_buffer_rsrc_t rnext = t + (int)gridDim.x < ntiles ? rw : make_rsrc(p.stream, 0);
+
+    // Inputs as B operand images: one x fragment per wave, one d fragment per
+    // wave 0 .. 3.  (The last reads of the previous tile's images lie before
+    // its last barrier.)
+    {
+      const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x + r0 * p.Kx, vrows * p.Kx * 2);
+      const int kb = wave & 3, rb = wave >> 2;
+      *(GP_LDS h8*)(mine + L_XI + img(kb, rb)) = input_frag(rx, 32 * rb + lr, p.Kx, kb, lh);
+      if (!TRUNK && wave < 4) {
+        const __amdgpu_buffer_rsrc_t rd = make_rsrc(p.d + r0 * p.Kd, vrows * p.Kd * 2);
+        const int kd = wave & 1, rd2 = wave >> 1;
+        *(GP_LDS h8*)(mine + L_DI + img(kd, rd2)) = input_frag(rd, 32 * rd2 + lr, p.Kd, kd, lh);
+      }
+      lds_barrier();
+    }
+
+    f16x acc[RB];
+    // One 256-wide layer's MFMAs: fragments J0 .. J0 + KB - 1, the first NX
+    // k-blocks from the x image, the others from image `src`; each fragment's
+    // register set is refilled with the one PF further on.
+    // The next layer's bias column (table offset nb, feature block nfb) is
+    // loaded meanwhile.
+    auto layer = [&](auto j0c, auto nxc, auto kbc, int src, int nb, int nfb) {
+      constexpr int J0 = decltype(j0c)::value, NX = decltype(nxc)::value, KB = decltype(kbc)::value;
+      const unsigned short b = bnext;
+      bnext = bias_at(nb, nfb);
+      h8 x[LB][RB];  // B operands, LB k-blocks ahead of their MFMAs
+      auto read = [&](auto kc) {
+        constexpr int kb = decltype(kc)::value;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          x[kb % LB][rb] = img_read(kb < NX ? mine + L_XI + img(kb, rb) : mine + src + img(kb - NX, rb));
+      };
+      static_for(std::make_integer_sequence<int, LB>{}, read);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) acc[rb] = biased(b);
+      static_for(std::make_integer_sequence<int, KB>{}, [&](auto kc) {
+        constexpr int kb = decltype(kc)::value, j = J0 + kb;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) acc[rb] = E::mma(wf[j % PF], x[kb % LB][rb], acc[rb]);
+        fetch(std::integral_constant<int, (j + PF) % T>{}, j + PF < T ? rw : rnext);
+        if constexpr (kb + LB < KB) read(std::integral_constant<int, kb + LB>{});
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    auto finish = [&](bool relu, int dst) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        h8 lo, hi;
+        to_operands<E>(acc[rb], relu, lo, hi);
+        *(GP_LDS h8*)(mine + dst + img(2 * wave, rb)) = lo;
+        *(GP_LDS h8*)(mine + dst + img(2 * wave + 1, rb)) = hi;
+      }
+      lds_barrier();
+    };
+    // Head: features 32 fb .. +31 of row block rb from image `src`, fragments
+    // hf (KB k-blocks), bias hb added in fp32, stored within the valid rows.
+    auto head = [&](const h8* hf, const h4* hb, auto kbc, int src, int fb, int rb, half_t* out, int N, int fn) {
+      constexpr int KB = decltype(kbc)::value;
+      f16x c = {};
+      static_for(std::make_integer_sequence<int, KB>{}, [&](auto kc) {
+        constexpr int kb = decltype(kc)::value;
+        c = E::mma(hf[kb], img_read(mine + src + kb * RB * FRAG + rb * FRAG), c);
+      });
+      const __amdgpu_buffer_rsrc_t ro = make_rsrc(out + r0 * N, vrows * N * 2);
+      const int row = 32 * rb + lr;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int f = 32 * fb + 8 * g + 4 * lh;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (f + e < N)
+            __builtin_amdgcn_raw_buffer_store_b16(
+                __builtin_bit_cast(unsigned short, E::cvt1(apply_act(c[4 * g + e] + E::val(hb[g][e]), fn))), ro,
+                (row * N + f + e) * 2, 0, 0);
+      }
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I4 = std::integral_constant<int, 4>;
+    using I8 = std::integral_constant<int, 8>;
+    using I16 = std::integral_constant<int, 16>;
+    using I20 = std::integral_constant<int, 20>;
+    constexpr int A = L_IMG, B = L_IMG + IMG;
+#define GP_J(j) std::integral_constant<int, j>{}
+    layer(GP_J(0), I4{}, I4{}, A, BF_L2, wave);
+    finish(true, A);
+    layer(GP_J(4), I0{}, I16{}, A, BF_L2 + 512, wave);
+    finish(true, B);
+    layer(GP_J(20), I0{}, I16{}, B, BF_L2 + 1024, wave);
+    finish(true, A);
+    layer(GP_J(36), I0{}, I16{}, A, BF_L2 + 1536, wave);
+    finish(true, B);
+    layer(GP_J(52), I0{}, I16{}, B, BF_L6, wave);
+    finish(true, A);
+    layer(GP_J(68), I4{}, I20{}, A, BF_L7, wave);
+    finish(true, B);
+    layer(GP_J(88), I0{}, I16{}, B, BF_L7 + 512, wave);
+    finish(true, A);
+    layer(GP_J(104), I0{}, I16{}, A, TRUNK ? BF_L1 : BF_L10, wave);
+    if constexpr (TRUNK) {
+      // Trunk output: the exchange and 16-byte stores of the 256-row kernel.
+      const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.out_r + r0 * 256, vrows * 256 * 2);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        u32x2 o[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          f4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaxf(acc[rb][4 * g + e], 0.f);
+          o[g] = __builtin_bit_cast(u32x2, E::cvt4(v));
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const auto x = __builtin_amdgcn_permlane32_swap(o[2 * q][0], o[2 * q + 1][0], false, false);
+          const auto y = __builtin_amdgcn_permlane32_swap(o[2 * q][1], o[2 * q + 1][1], false, false);
+          const u32x4 w = {(unsigned)x[0], (unsigned)y[0], (unsigned)x[1], (unsigned)y[1]};
+          buf_store_u4(ro, ((32 * rb + lr) * 256 + 32 * wave + 16 * q + 8 * lh) * 2, w);
+        }
+      }
+      lds_barrier();  // every wave has read this tile's images
+    } else {
+      finish(true, B);
+      // Layer 9 (density, from layer 8's image B) on waves 0 .. 3, one feature
+      // block and row block each, behind their layer 10; blocks past Na columns
+      // are skipped.
+      const int hfb = wave & 1, hrb = (wave >> 1) & 1;
+      const bool do9 = wave < 4 && 32 * hfb < p.Na, do12 = wave < 4 && 32 * hfb < p.Nrgb;
+      h8 hf[16];
+      h4 hb[4];
+      auto head_bias = [&](int off) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) hb[g] = buf_load_h4(rbias, (off + 32 * hfb + 8 * g + 4 * lh) * 2);
+      };
+      if (do9) {
+        head_bias(BH_L9);
+#pragma unroll
+        for (int kb = 0; kb < 16; ++kb) hf[kb] = load_frag(rw, 16 * lane + hfb * FRAG, S_L9 * SLOT + kb * 2 * FRAG);
+      }
+      layer(GP_J(120), I0{}, I16{}, B, BF_L11, wave & 3);
+      if (do9) head(hf, hb, I16{}, B, hfb, hrb, p.out_r, p.Na, ACT_NONE);
+      finish(false, A);
+      // Layer 11: [bottleneck | d] -> 128, wave w feature block w % 4 of row
+      // block w / 4; its output image goes into B.
+      if (do12) {
+        head_bias(BH_L12);
+#pragma unroll
+        for (int kb = 0; kb < 8; ++kb) hf[kb] = load_frag(rw, 16 * lane + hfb * FRAG, S_L12 * SLOT + kb * 2 * FRAG);
+      }
+      const int rb = wave >> 2;
+      f16x c = biased(bnext);
+      bnext = bias_at(BF_L1, wave);
+      static_for(std::make_integer_sequence<int, 18>{}, [&](auto kc) {
+        constexpr int k = decltype(kc)::value, j = kFour + k;
+        const h8 x = img_read((k < 2 ? mine + L_DI + k * RB * FRAG : mine + A + (k - 2) * RB * FRAG) + rb * FRAG);
+        c = E::mma(wf[j % PF], x, c);
+        fetch(std::integral_constant<int, (j + PF) % T>{}, j + PF < T ? rw : rnext);
+      });
+      h8 lo, hi;
+      to_operands<E>(c, true, lo, hi);
+      *(GP_LDS h8*)(mine + B + (2 * (wave & 3)) * RB * FRAG + rb * FRAG) = lo;
+      *(GP_LDS h8*)(mine + B + (2 * (wave & 3) + 1) * RB * FRAG + rb * FRAG) = hi;
+      lds_barrier();
+      // Layer 12 (colour) from image B; the next tile's first writes of B come
+      // after that tile's first barriers.
+      if (do12) head(hf, hb, I8{}, B, hfb, hrb, p.out_rgb, p.Nrgb, p.rgb_act);
+    }
+#undef GP_J
+  }
+  wait_vmcnt<0>();  // the fragments fetched past the last tile
+}
+}  // namespace split
+
 // ------------------------------------------------------------------ packing
 struct PackLayer {
   const half_t* w;  // [krows][n] (nn.Linear.weight.t())
@@ -557,6 +786,7 @@ struct PackLayer {
 };
 struct PackArgs {
   PackLayer L[12];
+  int n;  // layers, in slot order
   char* stream;
   half_t* bias;
 };
@@ -566,31 +796,30 @@ __global__ __launch_bounds__(256) void nerf_pack_kernel(PackArgs a) {
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
   constexpr int NFRAG_T = S_TOTAL * FPS * kWave;
   if (gid < NFRAG_T) {
-    const int s = gid / (FPS * kWave), pos = (gid / kWave) % FPS, lane = gid % kWave;
+    // A block packs four fragments of one slot, so the layer is the same for
+    // all of its threads: found with scalar compares against the slot map, and
+    // the eight loads of a thread are in flight together.
+    const int s = __builtin_amdgcn_readfirstlane(gid / (FPS * kWave));
+    const int pos = (gid / kWave) % FPS, lane = gid % kWave;
+    constexpr int first[11] = {S_L2, S_L2 + 8, S_L2 + 16, S_L2 + 24, S_L6, S_L7, S_L7 + 8, S_L9, S_L10, S_L11, S_L12};
+    int li = 0;
 #pragma unroll
-    for (int li = 0; li < 12; ++li) {
-      const PackLayer& L = a.L[li];
-      const int nslot = (L.kb * L.fb + FPS - 1) / FPS;
-      if (s < L.slot0 || s >= L.slot0 + nslot) continue;
-      const int fi = (s - L.slot0) * FPS + pos, kb = fi / L.fb, fb = fi % L.fb;
-      const int out = 32 * fb + (lane & 31), h = lane >> 5;
-      h8 v = {};
-      if (kb < L.kb && out < L.n) {
+    for (int i = 0; i < 11; ++i) li += s >= first[i];
+    if (li >= a.n) return;  // the trunk has no slots past layer 8
+    const PackLayer& L = a.L[li];
+    const int fi = (s - L.slot0) * FPS + pos, kb = fi / L.fb, fb = fi % L.fb;
+    const int out = 32 * fb + (lane & 31), h = lane >> 5;
+    const bool ok = kb < L.kb && out < L.n;
+    h8 v;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int pp = 8 * h + q;
-          int kin;
-          if (kb < L.next) {
-            const int c = 16 * kb + pp;
-            kin = c < L.ext_w ? L.ext_koff + c : -1;
-          } else {
-            kin = 16 * (kb - L.next) + sigma(pp);
-          }
-          v[q] = kin >= 0 ? L.w[(int64_t)kin * L.n + out] : (half_t)0.f;
-        }
-      }
-      *(h8*)(a.stream + (int64_t)s * SLOT + pos * FRAG + lane * 16) = v;
+    for (int q = 0; q < 8; ++q) {
+      const int pp = 8 * h + q, c = 16 * kb + pp;
+      const int kin = kb < L.next ? (c < L.ext_w ? L.ext_koff + c : -1) : 16 * (kb - L.next) + sigma(pp);
+      const bool in = ok && kin >= 0;
+      const half_t x = L.w[in ? (int64_t)kin * L.n + out : 0];
+      v[q] = in ? x : (half_t)0.f;
     }
+    *(h8*)(a.stream + (int64_t)s * SLOT + pos * FRAG + lane * 16) = v;
     return;
   }
   const int t = gid - NFRAG_T;
@@ -655,6 +884,18 @@ bool nerf_fused_supported(int64_t Kx, int64_t Kd, int64_t Na, int64_t Nrgb) {
   return Kx >= 1 && Kx <= 64 && Kd >= 1 && Kd <= 32 && Na >= 1 && Na <= 64 && Nrgb >= 1 && Nrgb <= 64;
 }
 
+// Rows of an M-row call, counted from its end, that run on the feature-split
+// kernel.  A 256-row tile takes 53 us (full chain, alone on its CU; 60 to 73
+// with all CUs busy) whatever part of it is valid, a 64-row split tile 18 to 23
+// us: calls of up to two rounds of split tiles (32,768 rows on 256 CUs: 42
+// against 60 us) are split whole, and so is what is left after the full rounds
+// of a larger call if it is no more than that; three rounds (62 us) are no
+// better than one of 256-row tiles.
+static int64_t split_rows(int64_t M, int num_cus) {
+  const int64_t rest = M % ((int64_t)num_cus * nerf::ROWS);
+  return rest <= 2 * (int64_t)num_cus * rows_split::ROWS ? rest : 0;
+}
+
 // Packs the weight stream and bias tables (all twelve layers, or the trunk's
 // first eight), then launches the fused kernel.
 static hipError_t fused_launch(bool trunk, int64_t M, int Kx, int Kd, int Na, int Nrgb, const void* x, const void* d,
@@ -683,28 +924,57 @@ static hipError_t fused_launch(bool trunk, int64_t M, int Kx, int Kd, int Na, in
                sh[8]};
   }
   // (The trunk's layers 9-12 stay zero: no slots, no bias entries.)
+  pa.n = nl;
   pa.stream = (char*)ws;
   pa.bias = (half_t*)((char*)ws + (size_t)S_TOTAL * SLOT);
   const int nthreads = S_TOTAL * FPS * kWave + B_TOTAL;
   hipLaunchKernelGGL(nerf_pack_kernel, dim3((nthreads + 255) / 256), dim3(256), 0, s, pa);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const Args a{(const half_t*)x, (const half_t*)d, (const char*)ws, pa.bias, (half_t*)out_r, (half_t*)out_rgb,
-               M, Kx, Kd, Na, Nrgb, rgb_act};
-  const int64_t tiles = (M + ROWS - 1) / ROWS;
-  const dim3 grid((unsigned)(tiles < num_cus ? tiles : num_cus));
-  if (trunk) {
-    if (dtype == GP_DTYPE_BF16)
-      hipLaunchKernelGGL((nerf_fused_kernel<BF16, true>), grid, dim3(NT), 0, s, a);
-    else
-      hipLaunchKernelGGL((nerf_fused_kernel<F16, true>), grid, dim3(NT), 0, s, a);
-  } else {
-    if (dtype == GP_DTYPE_BF16)
-      hipLaunchKernelGGL((nerf_fused_kernel<BF16, false>), grid, dim3(NT), 0, s, a);
-    else
-      hipLaunchKernelGGL((nerf_fused_kernel<F16, false>), grid, dim3(NT), 0, s, a);
+  Args a{(const half_t*)x, (const half_t*)d, (const char*)ws, pa.bias, (half_t*)out_r, (half_t*)out_rgb,
+         M, Kx, Kd, Na, Nrgb, rgb_act};
+  const int64_t few = split_rows(M, num_cus);
+  a.M = M - few;
+  if (a.M > 0) {
+    const int64_t tiles = (a.M + ROWS - 1) / ROWS;
+    const dim3 grid((unsigned)(tiles < num_cus ? tiles : num_cus));
+    if (trunk) {
+      if (dtype == GP_DTYPE_BF16)
+        hipLaunchKernelGGL((nerf_fused_kernel<BF16, true>), grid, dim3(NT), 0, s, a);
+      else
+        hipLaunchKernelGGL((nerf_fused_kernel<F16, true>), grid, dim3(NT), 0, s, a);
+    } else {
+      if (dtype == GP_DTYPE_BF16)
+        hipLaunchKernelGGL((nerf_fused_kernel<BF16, false>), grid, dim3(NT), 0, s, a);
+      else
+        hipLaunchKernelGGL((nerf_fused_kernel<F16, false>), grid, dim3(NT), 0, s, a);
+    }
+    if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  return hipGetLastError();
+  if (few > 0) {
+    // The rows before them are whole rounds of 256-row tiles, so x and d stay
+    // 16-byte aligned whatever their widths.
+    a.x += a.M * Kx;
+    a.d += a.d ? a.M * Kd : 0;
+    a.out_r += a.M * (trunk ? 256 : Na);
+    a.out_rgb += a.out_rgb ? a.M * Nrgb : 0;
+    a.M = few;
+    const int64_t tiles = (few + rows_split::ROWS - 1) / rows_split::ROWS;
+    const dim3 grid((unsigned)(tiles < num_cus ? tiles : num_cus)), block(rows_split::NT);
+    if (trunk) {
+      if (dtype == GP_DTYPE_BF16)
+        hipLaunchKernelGGL((split::nerf_split_kernel<BF16, true>), grid, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((split::nerf_split_kernel<F16, true>), grid, block, 0, s, a);
+    } else {
+      if (dtype == GP_DTYPE_BF16)
+        hipLaunchKernelGGL((split::nerf_split_kernel<BF16, false>), grid, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((split::nerf_split_kernel<F16, false>), grid, block, 0, s, a);
+    }
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 hipError_t nerf_fused_launch(int64_t M, int Kx, int Kd, int Na, int Nrgb, const void* x, const void* d,

@@ -300,3 +300,34 @@ def test_nerf_back_to_back_and_streams(cuda):
         assert_parity(f(r), wr, "rgb")
     assert torch.equal(a1.view(torch.int16), a3.view(torch.int16))
     assert torch.equal(r1.view(torch.int16), r3.view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Kx,Kd,Na,Nrgb", [(64, 27, 1, 3), (63, 32, 33, 4), (24, 5, 64, 64)])
+def test_nerf_few_rows_match_many(cuda, Kx, Kd, Na, Nrgb, dtype):
+    """Few rows run with the features split over the waves and 64 rows per
+    workgroup, full rounds of 256-row tiles with the rows split: the same
+    products in the same order, so the same bits, in the full chain and the
+    trunk.  Row counts around the edges of the 64-row tiles and of the rounds
+    (256 CUs: up to 32,768 rows are split, 65,536 are not, and of 65,536 + n the
+    last n are); input widths with and without whole 16-byte rows, heads on both
+    sides of one 32-feature block."""
+    M = 65536 + 32768
+    ws, bs = nerf_params(Kx, Kd, Na, Nrgb, seed=Kx, device=cuda, zero_pad_rows=None)
+    wb = [t.to(dtype) for p in zip(ws, bs) for t in p]
+    g = torch.Generator(device=cuda).manual_seed(1)
+    x = torch.rand((M, Kx), generator=g, device=cuda).to(dtype)
+    d = torch.rand((M, Kd), generator=g, device=cuda).to(dtype)
+    bits = lambda t: t.view(torch.int16)  # noqa: E731
+    big = gpipes.nerf_full(x[:65536], d[:65536], *wb, rgb_act="sigmoid") + (gpipes.nerf_a(x[:65536], *wb[:16]),)
+    for n in (1, 31, 33, 64, 65, 255, 4095, 20000, 32768, 32769):
+        a, c = gpipes.nerf_full(x[:n], d[:n], *wb, rgb_act="sigmoid")
+        h = gpipes.nerf_a(x[:n], *wb[:16])
+        for got, want in zip((a, c, h), big):
+            assert torch.equal(bits(got), bits(want[:n])), n
+    tail = gpipes.nerf_full(x[65536:], d[65536:], *wb, rgb_act="sigmoid") + (gpipes.nerf_a(x[65536:], *wb[:16]),)
+    for n in (1, 700, 32768):
+        m = 65536 + n
+        got = gpipes.nerf_full(x[:m], d[:m], *wb, rgb_act="sigmoid") + (gpipes.nerf_a(x[:m], *wb[:16]),)
+        for y, b, t in zip(got, big, tail):
+            assert torch.equal(bits(y[:65536]), bits(b)) and torch.equal(bits(y[65536:]), bits(t[:n])), m
