@@ -694,6 +694,249 @@ __global__ __launch_bounds__(256) void dlrm_tail_pack_kernel(TailPackArgs a) {
 }
 
 }  // namespace tail
+
+// ------------------------------------------------------------- few rows
+// Both chains with the features split over the waves and 64 rows per workgroup
+// (rows_split.hpp), from the same packed weights.
+namespace split {
+using rows_split::img;
+using rows_split::img_read;
+using rows_split::input_frag;
+using rows_split::load_frag;
+constexpr int RB = rows_split::RB, TR = rows_split::ROWS;
+constexpr int PF = 16;  // weight fragments in flight per wave
+constexpr int LB = 3;   // B operands are read from LDS this many k-blocks ahead
+
+// Rows of an M-row call, counted from its end, that run on a feature-split
+// kernel: calls of up to `rounds` rounds of 64-row tiles over the CUs, and as
+// much of what is left after the full rounds of 256-row tiles of larger ones.
+// Measured on 256 CUs (fp16, 256-row against split kernel, us):
+//   rows      bottom MLP   tail K 256    tail K 512    tail K 1024
+//    2,048   20.1 /  8.3   10.1 /  6.3   14.7 /  8.1   23.9 / 12.3
+//   16,384   22.3 / 10.2   10.5 /  7.7   15.9 / 11.4   27.0 / 18.2
+//   32,768   23.8 / 15.2   11.0 / 11.1   17.1 / 17.7   28.8 / 32.0
+//   49,152   23.3 / 21.8   11.1 / 13.8   18.8 / 23.6   31.3 / 45.3
+// so the bottom MLP takes two rounds (three would not pay for a launch of
+// their own behind a larger call), the tail one.
+static int64_t split_rows(int64_t M, int num_cus, int rounds) {
+  const int64_t rest = M % ((int64_t)num_cus * ROWS);
+  return rest <= rounds * (int64_t)num_cus * TR ? rest : 0;
+}
+
+// acc[rb] += W[kb] . B[kb] over k-blocks 0 .. KB-1 for NR row blocks: the
+// weight fragment of k-block kb is in wf[(J0 + kb) % PF], which refill(J0 + kb)
+// then loads anew; src(kb, rb) is the LDS address of the B operand.
+template <typename E, int J0, int KB, int NR, typename SRC, typename REFILL>
+__device__ __forceinline__ void layer(h8 (&wf)[PF], f16x (&acc)[NR], SRC src, REFILL refill) {
+  h8 x[LB][NR];
+  auto read = [&](auto kc) {
+    constexpr int kb = decltype(kc)::value;
+#pragma unroll
+    for (int rb = 0; rb < NR; ++rb) x[kb % LB][rb] = img_read(src(kb, rb));
+  };
+  static_for(std::make_integer_sequence<int, (LB < KB ? LB : KB)>{}, read);
+  static_for(std::make_integer_sequence<int, KB>{}, [&](auto kc) {
+    constexpr int kb = decltype(kc)::value;
+#pragma unroll
+    for (int rb = 0; rb < NR; ++rb) acc[rb] = E::mma(wf[(J0 + kb) % PF], x[kb % LB][rb], acc[rb]);
+    refill(std::integral_constant<int, J0 + kb>{});
+    if constexpr (kb + LB < KB) read(std::integral_constant<int, kb + LB>{});
+    __builtin_amdgcn_sched_barrier(0);
+  });
+}
+
+// The bottom MLP.  Wave w computes feature blocks w and w + 8 of the first
+// layer (fragments resident), block w of the second, and block w % 4 of row
+// block w / 4 of the third.
+template <typename E, int NKB1>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void dlrm_bot_split_kernel(Args p) {
+  constexpr int L_H1 = 0, L_H2 = L_H1 + 2 * FB1 * RB * FRAG, L_XI = L_H2 + 2 * FB2 * RB * FRAG;
+  constexpr int T = 2 * FB1 + KB3;  // streamed fragments per wave and tile
+  static_assert(T % PF == 0, "a tile's first fragment takes register set 0");
+  __shared__ __attribute__((aligned(1024))) char smem[L_XI + NKB1 * RB * FRAG];
+  const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  GP_LDS char* const mine = (GP_LDS char*)smem + 16 * lane;
+  const int ntiles = (int)((p.M + TR - 1) / TR);
+
+  const __amdgpu_buffer_rsrc_t rp = make_rsrc(p.pack, (int)P_TOTAL), none = make_rsrc(p.pack, 0);
+  const int v8 = 16 * lane + wave * FRAG, v4 = 16 * lane + (wave & 3) * FRAG;
+  h8 wf[PF], w1[2][NKB1];
+  // Streamed fragment j: k-block j of the second layer, then of the third.
+  auto fetch = [&](auto jc, __amdgpu_buffer_rsrc_t r) {
+    constexpr int j = decltype(jc)::value, j3 = j - 2 * FB1;
+    constexpr int off = (int)P_STREAM + (j3 < 0 ? j * FB2 * FRAG : S_W3 * SLOT + j3 * FB3 * FRAG);
+    wf[j % PF] = load_frag(r, j3 < 0 ? v8 : v4, off);
+  };
+  auto bias_at = [&](int off, int fb) {  // A operand: the bias at k = 0
+    h8 a = {};
+    a[0] = __builtin_bit_cast(half_t, (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(
+                                          rp, (int)P_BIAS + (off + 64 * fb + lane) * 2, 0, 0));
+    return a;
+  };
+  h8 ones = {};
+  ones[0] = __builtin_bit_cast(half_t, lane < 32 ? E::kOne : (unsigned short)0);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int kb = 0; kb < NKB1; ++kb) w1[i][kb] = load_frag(rp, 16 * lane, (2 * (wave + 8 * i) + kb) * FRAG);
+  const h8 b1[2] = {bias_at(BF_1, wave), bias_at(BF_1, wave + 8)}, b2 = bias_at(BF_2, wave),
+           b3 = bias_at(BF_3, wave & 3);
+  static_for(std::make_integer_sequence<int, PF>{}, [&](auto j) { fetch(j, rp); });
+
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const int64_t r0 = (int64_t)t * TR;
+    const int vrows = p.M - r0 < TR ? (int)(p.M - r0) : TR;
+    // Past the last tile the next tile's fragments come through an empty
+    // descriptor.
+    const __amdgpu_buffer_rsrc_t rnext = t + (int)gridDim.x < ntiles ? rp : none;
+    auto refill = [&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      fetch(std::integral_constant<int, (j + PF) % T>{}, j + PF < T ? rp : rnext);
+    };
+    if (wave < NKB1 * RB) {
+      const int kb = wave / RB, rb = wave % RB;
+      const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x + r0 * p.K0, vrows * p.K0 * 2);
+      *(GP_LDS h8*)(mine + L_XI + img(kb, rb)) = input_frag(rx, 32 * rb + lr, p.K0, kb, lh);
+    }
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        f16x c = E::mma(b1[i], ones, f16x{});
+#pragma unroll
+        for (int kb = 0; kb < NKB1; ++kb) c = E::mma(w1[i][kb], img_read(mine + L_XI + img(kb, rb)), c);
+        h8 lo, hi;
+        to_operands<E>(c, p.relu1 != 0, lo, hi);
+        *(GP_LDS h8*)(mine + L_H1 + img(2 * (wave + 8 * i), rb)) = lo;
+        *(GP_LDS h8*)(mine + L_H1 + img(2 * (wave + 8 * i) + 1, rb)) = hi;
+      }
+    lds_barrier();
+    f16x acc[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) acc[rb] = E::mma(b2, ones, f16x{});
+    layer<E, 0, 2 * FB1, RB>(wf, acc, [&](int kb, int rb) { return mine + L_H1 + img(kb, rb); }, refill);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      h8 lo, hi;
+      to_operands<E>(acc[rb], p.relu2 != 0, lo, hi);
+      *(GP_LDS h8*)(mine + L_H2 + img(2 * wave, rb)) = lo;
+      *(GP_LDS h8*)(mine + L_H2 + img(2 * wave + 1, rb)) = hi;
+    }
+    lds_barrier();
+    const int rb3 = wave >> 2, fb3 = wave & 3;
+    f16x c3[1] = {E::mma(b3, ones, f16x{})};
+    layer<E, 2 * FB1, KB3, 1>(wf, c3, [&](int kb, int) { return mine + L_H2 + kb * RB * FRAG + rb3 * FRAG; }, refill);
+    // Output: the exchange and 16-byte stores of the 256-row kernel.
+    const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.out + r0 * H3, vrows * H3 * 2);
+    u32x2 o[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = apply_act(c3[0][4 * g + e], p.act3);
+      o[g] = __builtin_bit_cast(u32x2, E::cvt4(v));
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const auto x = __builtin_amdgcn_permlane32_swap(o[2 * q][0], o[2 * q + 1][0], false, false);
+      const auto y = __builtin_amdgcn_permlane32_swap(o[2 * q][1], o[2 * q + 1][1], false, false);
+      const u32x4 w = {(unsigned)x[0], (unsigned)y[0], (unsigned)x[1], (unsigned)y[1]};
+      buf_store_u4(ro, ((32 * rb3 + lr) * H3 + 32 * fb3 + 16 * q + 8 * lh) * 2, w);
+    }
+    // (The next tile's writes: of the x image after two barriers every wave
+    // passed since reading it, of the first layer's image after one, of the
+    // second layer's after that tile's first two.)
+  }
+  wait_vmcnt<0>();  // the fragments fetched past the last tile
+}
+
+// The top MLP's tail: K -> 256 with wave w on feature block w, then the click
+// head on waves 0 .. RB - 1, one row block each, over the hidden image in the
+// 256-row kernel's order.
+template <typename E, int ST>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void dlrm_tail_split_kernel(
+    tail::TailArgs p) {
+  constexpr int K = 32 * ST, KB = K / 16;
+  // (At K = 1024 the input image fills the LDS: the hidden image takes its
+  // place, between two more barriers.)
+  constexpr bool OVER = KB * RB * FRAG > 96 * 1024;
+  constexpr int L_XI = 0, L_H = OVER ? L_XI : KB * RB * FRAG, L_W = KB * RB * FRAG + (OVER ? 0 : 2 * FB2 * RB * FRAG);
+  static_assert(KB % PF == 0 && L_W + H2 * 4 <= 160 * 1024, "register sets / LDS");
+  __shared__ __attribute__((aligned(1024))) char smem[L_W + H2 * 4];
+  const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  GP_LDS char* const mine = (GP_LDS char*)smem + 16 * lane;
+  GP_LDS float* const w5 = (GP_LDS float*)(smem + L_W);
+  const int ntiles = (int)((p.M + TR - 1) / TR);
+
+  const __amdgpu_buffer_rsrc_t rp = make_rsrc(p.pack, (int)tail::p_total(ST)), none = make_rsrc(p.pack, 0);
+  h8 wf[PF];
+  auto fetch = [&](auto jc, __amdgpu_buffer_rsrc_t r) {
+    constexpr int j = decltype(jc)::value;
+    wf[j % PF] = load_frag(r, 16 * lane + wave * FRAG, j * FB2 * FRAG);
+  };
+  const half_t* const bias = (const half_t*)(p.pack + tail::p_bias(ST));
+  const float* const head = (const float*)(p.pack + tail::p_head(ST));
+  h8 b4 = {}, ones = {};
+  b4[0] = bias[64 * wave + lane];
+  ones[0] = __builtin_bit_cast(half_t, lane < 32 ? E::kOne : (unsigned short)0);
+  if (threadIdx.x < H2) w5[threadIdx.x] = head[threadIdx.x];
+  const float b5 = head[H2];
+  static_for(std::make_integer_sequence<int, PF>{}, [&](auto j) { fetch(j, rp); });
+
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    const int64_t r0 = (int64_t)t * TR;
+    const int vrows = p.M - r0 < TR ? (int)(p.M - r0) : TR;
+    const __amdgpu_buffer_rsrc_t rnext = t + (int)gridDim.x < ntiles ? rp : none;
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x + r0 * K, vrows * K * 2);
+#pragma unroll
+    for (int i = 0; i < KB * RB / NW; ++i) {
+      const int f = NW * i + wave, kb = f / RB, rb = f % RB;
+      *(GP_LDS h8*)(mine + L_XI + img(kb, rb)) = load_frag(rx, ((32 * rb + lr) * K + 16 * kb + 8 * lh) * 2, 0);
+    }
+    lds_barrier();
+    f16x acc[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) acc[rb] = E::mma(b4, ones, f16x{});
+    layer<E, 0, KB, RB>(wf, acc, [&](int kb, int rb) { return mine + L_XI + img(kb, rb); }, [&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      fetch(std::integral_constant<int, (j + PF) % KB>{}, j + PF < KB ? rp : rnext);
+    });
+    if constexpr (OVER) lds_barrier();
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      h8 lo, hi;
+      to_operands<E>(acc[rb], p.relu != 0, lo, hi);
+      *(GP_LDS h8*)(mine + L_H + img(2 * wave, rb)) = lo;
+      *(GP_LDS h8*)(mine + L_H + img(2 * wave + 1, rb)) = hi;
+    }
+    lds_barrier();
+    if (wave < RB) {
+      float sum = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < 2 * FB2; ++kb) {
+        const h8 v = img_read(mine + L_H + kb * RB * FRAG + wave * FRAG);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          const f4 w = *(GP_LDS const f4*)(w5 + 16 * kb + 8 * g + 4 * lh);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum = __builtin_fmaf(E::val(v[4 * g + e]), w[e], sum);
+        }
+      }
+      sum = sum_lane_halves(sum);
+      const unsigned short o = __builtin_bit_cast(unsigned short, E::cvt1(apply_act(sum + b5, p.act_out)));
+      const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.out + r0, vrows * 2);
+      __builtin_amdgcn_raw_buffer_store_b16(o, ro, lh == 0 ? 2 * (32 * wave + lr) : 2 * TR, 0, 0);
+    }
+    // (The hidden image is written again only after the next tile's first
+    // barrier.)
+    if constexpr (OVER) lds_barrier();
+  }
+  wait_vmcnt<0>();  // the fragments fetched past the last tile
+}
+}  // namespace split
 }  // namespace dlrm
 
 size_t dlrm_tail_workspace(int64_t K) { return dlrm::tail::p_total((int)(K / 32)); }
@@ -718,21 +961,36 @@ hipError_t dlrm_tail_launch(int64_t M, int64_t K, const void* x, const void* w4,
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  const TailArgs a{(const half_t*)x, (const char*)ws, (half_t*)out, M, act4 == GP_ACT_RELU, act5};
-  const int64_t tiles = (M + ROWS - 1) / ROWS;
-  const dim3 grid((unsigned)(tiles < num_cus ? tiles : num_cus));
-#define GP_TAIL(T, S) hipLaunchKernelGGL((dlrm_tail_kernel<T, S>), grid, dim3(NT), 0, s, a)
-  if (dtype == GP_DTYPE_BF16) {
-    if (ST == 8) GP_TAIL(BF16, 8);
-    else if (ST == 16) GP_TAIL(BF16, 16);
-    else GP_TAIL(BF16, 32);
-  } else {
-    if (ST == 8) GP_TAIL(F16, 8);
-    else if (ST == 16) GP_TAIL(F16, 16);
-    else GP_TAIL(F16, 32);
+  TailArgs a{(const half_t*)x, (const char*)ws, (half_t*)out, M, act4 == GP_ACT_RELU, act5};
+  auto go = [&](auto type, auto slots, bool few) {
+    using E = decltype(type);
+    constexpr int S = decltype(slots)::value;
+    const int64_t tr = few ? split::TR : ROWS, tiles = (a.M + tr - 1) / tr;
+    const dim3 grid((unsigned)(tiles < num_cus ? tiles : num_cus));
+    if (few)
+      hipLaunchKernelGGL((split::dlrm_tail_split_kernel<E, S>), grid, dim3(NT), 0, s, a);
+    else
+      hipLaunchKernelGGL((dlrm_tail_kernel<E, S>), grid, dim3(NT), 0, s, a);
+    return hipGetLastError();
+  };
+  auto run = [&](bool few) {
+    using S8 = std::integral_constant<int, 8>;
+    using S16 = std::integral_constant<int, 16>;
+    using S32 = std::integral_constant<int, 32>;
+    if (dtype == GP_DTYPE_BF16) return ST == 8 ? go(BF16{}, S8{}, few) : ST == 16 ? go(BF16{}, S16{}, few) : go(BF16{}, S32{}, few);
+    return ST == 8 ? go(F16{}, S8{}, few) : ST == 16 ? go(F16{}, S16{}, few) : go(F16{}, S32{}, few);
+  };
+  const int64_t few = split::split_rows(M, num_cus, 1);
+  hipError_t e = hipSuccess;
+  a.M = M - few;
+  if (a.M > 0) e = run(false);
+  if (few > 0 && e == hipSuccess) {
+    a.x += a.M * K;
+    a.out += a.M;
+    a.M = few;
+    e = run(true);
   }
-#undef GP_TAIL
-  return hipGetLastError();
+  return e;
 }
 
 size_t dlrm_bot_workspace() { return dlrm::P_TOTAL; }
@@ -750,23 +1008,36 @@ hipError_t dlrm_bot_launch(int64_t M, int K0, const void* x, const void* const* 
   hipLaunchKernelGGL(dlrm_pack_kernel, dim3((nthreads + 255) / 256), dim3(256), 0, s, pa);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const Args a{(const half_t*)x, (const char*)ws, (half_t*)out, M, K0,
-               acts[0] == GP_ACT_RELU, acts[1] == GP_ACT_RELU, acts[2]};
-  const int64_t tiles = (M + ROWS - 1) / ROWS;
-  const dim3 grid((unsigned)(tiles < num_cus ? tiles : num_cus));
-  const bool two = K0 > 16;
-  if (dtype == GP_DTYPE_BF16) {
-    if (two)
-      hipLaunchKernelGGL((dlrm_bot_kernel<BF16, 2>), grid, dim3(NT), 0, s, a);
+  Args a{(const half_t*)x, (const char*)ws, (half_t*)out, M, K0,
+         acts[0] == GP_ACT_RELU, acts[1] == GP_ACT_RELU, acts[2]};
+  auto go = [&](auto type, auto nkb, bool few) {
+    using E = decltype(type);
+    constexpr int N = decltype(nkb)::value;
+    const int64_t tr = few ? split::TR : ROWS, tiles = (a.M + tr - 1) / tr;
+    const dim3 grid((unsigned)(tiles < num_cus ? tiles : num_cus));
+    if (few)
+      hipLaunchKernelGGL((split::dlrm_bot_split_kernel<E, N>), grid, dim3(NT), 0, s, a);
     else
-      hipLaunchKernelGGL((dlrm_bot_kernel<BF16, 1>), grid, dim3(NT), 0, s, a);
-  } else {
-    if (two)
-      hipLaunchKernelGGL((dlrm_bot_kernel<F16, 2>), grid, dim3(NT), 0, s, a);
-    else
-      hipLaunchKernelGGL((dlrm_bot_kernel<F16, 1>), grid, dim3(NT), 0, s, a);
+      hipLaunchKernelGGL((dlrm_bot_kernel<E, N>), grid, dim3(NT), 0, s, a);
+    return hipGetLastError();
+  };
+  auto run = [&](bool few) {
+    using N1 = std::integral_constant<int, 1>;
+    using N2 = std::integral_constant<int, 2>;
+    if (dtype == GP_DTYPE_BF16) return K0 > 16 ? go(BF16{}, N2{}, few) : go(BF16{}, N1{}, few);
+    return K0 > 16 ? go(F16{}, N2{}, few) : go(F16{}, N1{}, few);
+  };
+  const int64_t few = split::split_rows(M, num_cus, 2);
+  a.M = M - few;
+  if (a.M > 0) e = run(false);
+  if (few > 0 && e == hipSuccess) {
+    // whole rounds of 256 rows before them: x and out stay 16-byte aligned
+    a.x += a.M * K0;
+    a.out += a.M * H3;
+    a.M = few;
+    e = run(true);
   }
-  return hipGetLastError();
+  return e;
 }
 
 }  // namespace gp

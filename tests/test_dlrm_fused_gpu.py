@@ -254,3 +254,39 @@ def test_dlrm_fused_randomized_sweep(cuda):
         print(f"[dlrm-tail] sweep {i}: K={K} M={M} acts={acts} bias={bias} {dtype}", flush=True)
         y, want, *_ = run_tail(cuda, M, [K, 256, 1], acts, seed=200 + i, bias=bias, dtype=dtype)
         check(f(y), want, f"tail sweep {i}", bf16=dtype == BF)
+
+
+# ------------------------------------------------------------------ few rows
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_dlrm_few_rows_match_many(cuda, dtype):
+    """Few rows run with the features split over the waves and 64 rows per
+    workgroup, full rounds of 256-row tiles with the rows split: the same
+    products in the same order, so the same bits.  Row counts around the edges
+    of the 64-row tiles and of the rounds (on 256 CUs the bottom MLP is split up
+    to 32,768 rows, the tail up to 16,384, and so are the last n of 65,536 + n);
+    first layers of one and two k-blocks, odd and even widths; tails of each K."""
+    g = torch.Generator(device=cuda).manual_seed(5)
+
+    def lin(k, n):
+        return ((torch.randn(k, n, generator=g, device=cuda) / k ** 0.5).to(dtype),
+                (torch.randn(n, generator=g, device=cuda) * 0.3).to(dtype))
+
+    bits = lambda t: t.view(torch.int16)  # noqa: E731
+    M = 65536 + 20000
+
+    def check(call, x):
+        big, rest = call(x[:65536]), call(x[65536:])
+        for n in (1, 33, 64, 65, 255, 4097, 16384, 16385, 32768, 32769):
+            assert torch.equal(bits(call(x[:n])), bits(big[:n])), n
+        for n in (1, 500, 16384, 20000):
+            y = call(x[:65536 + n])
+            assert torch.equal(bits(y[:65536]), bits(big)) and torch.equal(bits(y[65536:]), bits(rest[:n])), n
+
+    for K0 in (13, 16, 27):
+        ws, bs = zip(*(lin(k, n) for k, n in ((K0, 512), (512, 256), (256, 128))))
+        x = torch.rand((M, K0), generator=g, device=cuda).to(dtype)
+        check(lambda v: gpipes.mlp_out(v, ws, bs, ["relu"] * 3), x)
+    for K in (256, 512, 1024):
+        ws, bs = zip(*(lin(k, n) for k, n in ((K, 256), (256, 1))))
+        x = torch.randn((M, K), generator=g, device=cuda).to(dtype)
+        check(lambda v: gpipes.mlp_out(v, ws, bs, ["relu", "sigmoid"]), x)
