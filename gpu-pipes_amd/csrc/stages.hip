@@ -473,17 +473,47 @@ __global__ __launch_bounds__(kStageThreads) void place_kernel(const half_t* src,
   }
 }
 
+// The same without an activation for a source whose rows are not whole
+// 16-byte chunks (a width of 479, say) into a 16-byte aligned destination: one
+// thread per eight destination columns, its eight 2-byte loads in flight
+// together, one 16-byte store.  The source is read once through L1 either way;
+// against one element per thread (place_kernel<1>) this takes an eighth of the
+// threads, index divisions and stores.
+__global__ __launch_bounds__(kStageThreads) void place_rows_kernel(const unsigned short* src, int64_t lds, int w,
+                                                                   unsigned short* dst, int64_t ldd, int wpad,
+                                                                   int64_t M) {
+  typedef unsigned short us8 __attribute__((ext_vector_type(8)));
+  const int vpr = wpad / 8;
+  const int64_t total = M * vpr;
+  for (int64_t i = (int64_t)blockIdx.x * kStageThreads + threadIdx.x; i < total;
+       i += (int64_t)gridDim.x * kStageThreads) {
+    const int64_t m = i / vpr;
+    const int j = (int)(i - m * vpr) * 8;
+    const unsigned short* const r = src + m * lds;
+    us8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = r[j + e < w ? j + e : 0];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = j + e < w ? v[e] : (unsigned short)0;
+    *(us8*)(dst + m * ldd + j) = v;
+  }
+}
+
 hipError_t place_launch(int64_t M, const void* src, int64_t lds, int64_t w, void* dst, int64_t ldd, int64_t wpad,
                         int act, int num_cus, hipStream_t s) {
   if (M <= 0 || wpad <= 0) return hipSuccess;
   const bool vec = wpad % 8 == 0 && ldd % 8 == 0 && ((uintptr_t)dst & 15) == 0 &&
                    (w == 0 || (w % 8 == 0 && lds % 8 == 0 && ((uintptr_t)src & 15) == 0));
-  const int V = vec ? 8 : 1;
+  const bool rows = !vec && act == ACT_NONE && w > 0 && wpad % 8 == 0 && ldd % 8 == 0 && ((uintptr_t)dst & 15) == 0;
+  const int V = vec || rows ? 8 : 1;
   const int64_t want = (M * (wpad / V) + kStageThreads - 1) / kStageThreads, cap = (int64_t)num_cus * 16;
   const dim3 grid((unsigned)(want < cap ? want : cap)), block(kStageThreads);
   if (vec)
     hipLaunchKernelGGL(place_kernel<8>, grid, block, 0, s, (const half_t*)src, lds, (int)w, (half_t*)dst, ldd,
                        (int)wpad, act, M);
+  else if (rows)
+    hipLaunchKernelGGL(place_rows_kernel, grid, block, 0, s, (const unsigned short*)src, lds, (int)w,
+                       (unsigned short*)dst, ldd, (int)wpad, M);
   else
     hipLaunchKernelGGL(place_kernel<1>, grid, block, 0, s, (const half_t*)src, lds, (int)w, (half_t*)dst, ldd,
                        (int)wpad, act, M);

@@ -290,3 +290,22 @@ def test_dlrm_few_rows_match_many(cuda, dtype):
         ws, bs = zip(*(lin(k, n) for k, n in ((K, 256), (256, 1))))
         x = torch.randn((M, K), generator=g, device=cuda).to(dtype)
         check(lambda v: gpipes.mlp_out(v, ws, bs, ["relu", "sigmoid"]), x)
+
+
+@pytest.mark.parametrize("K", [3, 479, 513])
+def test_mlp_unaligned_rows_padded(cuda, K):
+    """Input rows that are not whole 16-byte chunks are padded eight columns to a
+    thread; bits as from an input padded beforehand, also from an unaligned base."""
+    M, N = 1003, 256
+    Kp = (K + 7) // 8 * 8
+    g = torch.Generator(device=cuda).manual_seed(K)
+    w = torch.zeros((Kp, N), dtype=torch.float16, device=cuda)
+    w[:K] = (torch.randn((K, N), generator=g, device=cuda) / K ** 0.5).half()
+    b = torch.randn(N, generator=g, device=cuda).half()
+    flat = torch.randn(M * K + 1, generator=g, device=cuda).half()
+    for off in (0, 1):
+        x = flat[off:off + M * K].view(M, K)
+        xp = torch.zeros((M, Kp), dtype=torch.float16, device=cuda)
+        xp[:, :K] = x
+        got = gpipes.mlp_out(x, [w[:K].contiguous()], [b], ["relu"])
+        assert torch.equal(got.view(torch.int16), gpipes.mlp_out(xp, [w], [b], ["relu"]).view(torch.int16))
