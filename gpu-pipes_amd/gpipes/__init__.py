@@ -127,12 +127,53 @@ def _check(rc):
         raise GpipesError(rc, lib.gp_last_error().decode())
 
 
-def _stream_ptr(t):
+# The allocating forms leave their outputs uninitialised (the reference zeroes
+# them): the kernels write every row, and the fill was a pass over the output --
+# 14 us of the 57 us that a 262,144-row MGN node MLP took.
+#
+# The host side of a call: about thirty attribute checks, a device guard and a
+# stream lookup.  torch.cuda.device() and torch.cuda.current_stream() cost
+# several microseconds a call, as long as a small kernel runs, so the guard below
+# touches the device only when it has to change, and the raw stream handle is
+# asked for directly where torch has the function for it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+class _on:
+    """Makes a tensor's device current for the block (as torch.cuda.device(t.device))."""
+
+    __slots__ = ("dev", "prev")
+
+    def __init__(self, t):
+        self.dev = t.get_device()
+
+    def __enter__(self):
+        self.prev = torch.cuda.current_device()
+        if self.prev != self.dev:
+            torch.cuda.set_device(self.dev)
+
+    def __exit__(self, *exc):
+        if self.prev != self.dev:
+            torch.cuda.set_device(self.prev)
+
+
+def _stream(t):
+    """Handle of torch's current stream on the tensor's device."""
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def _ok(t, shape, dtype):
+    """Whether t passes _check_input(name, t, shape, dtype)."""
+    return (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is dtype and t.is_contiguous()
+            and (shape is None or t.shape == shape))
 
 
 def _check_input(name, t, shape=None, dtype=torch.float16):
     # CHECK_CUDA / CHECK_CONTIGUOUS of mgn_fullmlp_pl_ext.cu:14-16, plus dtype/shape
+    if _ok(t, shape, dtype):
+        return
     if not isinstance(t, torch.Tensor):
         raise RuntimeError(f"{name} must be a torch.Tensor")
     if not t.is_cuda:
@@ -141,12 +182,31 @@ def _check_input(name, t, shape=None, dtype=torch.float16):
         raise RuntimeError(f"{name} must be contiguous")
     if t.dtype != dtype:
         raise RuntimeError(f"{name} must be {str(dtype).replace('torch.', '')} (got {t.dtype})")
-    if shape is not None and tuple(t.shape) != tuple(shape):
-        raise RuntimeError(f"{name} must have shape {tuple(shape)} (got {tuple(t.shape)})")
+    raise RuntimeError(f"{name} must have shape {tuple(shape)} (got {tuple(t.shape)})")
+
+
+def _check_layers(ws, bs, shapes, dtype):
+    """Weights w1, w2, ... of the given [in, out] shapes and their optional biases."""
+    for i, (w, b, shp) in enumerate(zip(ws, bs, shapes)):
+        if not _ok(w, shp, dtype):
+            _check_input(f"w{i + 1}", w, shp, dtype)
+        if b is not None and not _ok(b, shp[1:], dtype):
+            _check_input(f"b{i + 1}", b, shp[1:], dtype)
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+def _same_device(*ts):
+    dev = None
+    for t in ts:
+        if t is not None:
+            d = t.get_device()
+            if dev is None:
+                dev = d
+            elif d != dev:
+                raise RuntimeError("all tensors must be on the same device")
 
 
 _DTYPES = {torch.float16: 0, torch.bfloat16: 1}  # GP_DTYPE_F16, GP_DTYPE_BF16
@@ -176,23 +236,21 @@ def mgn_mlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps=1e-5, impl="fus
         _check_input("gamma", gamma, (128,), dt)
         _check_input("beta", beta, (128,), dt)
     _check_input("out", out, (M, 128), dt)
-    devs = {t.device for t in (x, w1, b1, w2, b2, w3, b3, out) if t is not None}
-    if len(devs) != 1:
-        raise RuntimeError("all tensors must be on the same device")
+    _same_device(x, w1, b1, w2, b2, w3, b3, out)
     impl_id = _IMPLS.get(impl, impl)
-    with torch.cuda.device(x.device):
+    with _on(x):
         args = (M, K, _ptr(x), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(w3), _ptr(b3), _ptr(gamma),
                 _ptr(beta), float(eps), _ptr(out), int(impl_id))
         if dt == torch.float16:
-            rc = lib.gp_mgn_mlp_out(*args, ctypes.c_void_p(_stream_ptr(x)))
+            rc = lib.gp_mgn_mlp_out(*args, _stream(x))
         else:
-            rc = lib.gp_mgn_mlp_dtype_out(*args, _DTYPES[dt], ctypes.c_void_p(_stream_ptr(x)))
+            rc = lib.gp_mgn_mlp_dtype_out(*args, _DTYPES[dt], _stream(x))
     _check(rc)
     return out
 
 
 def mgn_mlp(x, w1, b1, w2, b2, w3, b3, gamma=None, beta=None, eps=1e-5, impl="fused"):
-    out = torch.zeros((x.shape[0], 128), dtype=x.dtype, device=x.device)
+    out = torch.empty((x.shape[0], 128), dtype=x.dtype, device=x.device)
     return mgn_mlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps=eps, impl=impl)
 
 
@@ -207,7 +265,7 @@ def mgn_fullmlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out):
 
 def mgn_fullmlp(x, w1, b1, w2, b2, w3, b3, gamma, beta):
     """Allocating form: returns a new [M, 128] tensor (mgn_fullmlp_pl_ext.cu:74-88)."""
-    out = torch.zeros((x.shape[0], 128), dtype=x.dtype, device=x.device)
+    out = torch.empty((x.shape[0], 128), dtype=x.dtype, device=x.device)
     return mgn_fullmlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out)
 
 
@@ -220,7 +278,7 @@ def mgn_linears_out(x, w1, b1, w2, b2, w3, b3, out):
 
 
 def mgn_linears(x, w1, b1, w2, b2, w3, b3):
-    out = torch.zeros((x.shape[0], 128), dtype=x.dtype, device=x.device)
+    out = torch.empty((x.shape[0], 128), dtype=x.dtype, device=x.device)
     return mgn_linears_out(x, w1, b1, w2, b2, w3, b3, out)
 
 
@@ -240,10 +298,6 @@ def _dtype_of(x):
     return x.dtype if isinstance(x, torch.Tensor) and x.dtype in _DTYPES else torch.float16
 
 
-def _stream(t):
-    return ctypes.c_void_p(_stream_ptr(t))
-
-
 def linear_out(x, w, b=None, acc=None, act="none", out=None):
     """out[M,128] = act(x @ w + b [+ acc]) -- pipe_gemm_bias_relu / pipe_gemm_bias / pipe_gemm."""
     _check_input("x", x)
@@ -254,7 +308,7 @@ def linear_out(x, w, b=None, acc=None, act="none", out=None):
     if out is None:
         out = torch.empty((M, 128), dtype=torch.float16, device=x.device)
     _check_input("out", out, (M, 128))
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_linear_out(M, K, _ptr(x), _ptr(w), _ptr(b), _ptr(acc), ACTS.get(act, act), _ptr(out),
                                  _stream(x)))
     return out
@@ -271,7 +325,7 @@ def linear_layer_norm_out(x, w, b, gamma, beta, eps=1e-5, out=None):
     if out is None:
         out = torch.empty((M, 128), dtype=torch.float16, device=x.device)
     _check_input("out", out, (M, 128))
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_linear_layer_norm_out(M, K, _ptr(x), _ptr(w), _ptr(b), _ptr(gamma), _ptr(beta), float(eps),
                                             _ptr(out), _stream(x)))
     return out
@@ -286,7 +340,7 @@ def layer_norm_out(x, gamma=None, beta=None, eps=1e-5, out=None):
     if out is None:
         out = torch.empty_like(x)
     _check_input("out", out, (M, D))
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_layer_norm_out(M, D, _ptr(x), _ptr(gamma), _ptr(beta), float(eps), _ptr(out), _stream(x)))
     return out
 
@@ -299,7 +353,7 @@ def add_out(a, b, out=None):
     if out is None:
         out = torch.empty_like(a)
     _check_input("out", out, (M, N))
-    with torch.cuda.device(a.device):
+    with _on(a):
         _check(lib.gp_add_out(M, N, _ptr(a), _ptr(b), _ptr(out), _stream(a)))
     return out
 
@@ -315,7 +369,7 @@ def concat_out(a, b, out=None):
     if out is None:
         out = torch.empty((M, N0 + N1), dtype=a.dtype, device=a.device)
     _check_input("out", out, (M, N0 + N1))
-    with torch.cuda.device(a.device):
+    with _on(a):
         _check(lib.gp_concat_out(M, N0, N1, _ptr(a), _ptr(b), _ptr(out), _stream(a)))
     return out
 
@@ -329,7 +383,7 @@ def pipe_ident(x, max_pipes=0, out=None):
     if out is None:
         out = torch.zeros_like(x)
     _check_input("out", out, (M, D))
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_pipe_ident(M, _ptr(x), _ptr(out), int(max_pipes), _stream(x)))
     return out
 
@@ -345,7 +399,7 @@ def pipe_route(x, route="ident", max_pipes=0):
     rid = ROUTES.get(route, route)
     out = torch.zeros_like(x)
     out2 = torch.zeros_like(x) if rid == ROUTES["broadcast"] else None
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_pipe_route(M, _ptr(x), _ptr(out), _ptr(out2), int(rid), int(max_pipes), _stream(x)))
     return out, out2
 
@@ -361,7 +415,7 @@ def pipe_handoff(M, max_pipes=0, device=None, out=None):
         out = torch.zeros(max(T, 1), dtype=torch.int32, device=dev)
     if out.dtype != torch.int32 or not out.is_cuda or out.numel() < T or not out.is_contiguous():
         raise RuntimeError("out must be a contiguous int32 CUDA tensor of ceil(M / 128) elements")
-    with torch.cuda.device(out.device):
+    with _on(out):
         _check(lib.gp_pipe_route(int(M), None, _ptr(out), None, ROUTES["handoff"], int(max_pipes), _stream(out)))
     return out
 
@@ -420,9 +474,9 @@ def fill_normal(t, seed=0, offset=0):
     as oracle.normal on the host), on the current stream; returns t."""
     if not t.is_cuda or not t.is_contiguous():
         raise GpipesError("fill_normal needs a contiguous CUDA tensor")
-    with torch.cuda.device(t.device):
+    with _on(t):
         _check(lib.gp_fill_normal(_ptr(t), t.numel(), int(seed), int(offset), _DTYPES.get(t.dtype, -1),
-                                  ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)))
+                                  _stream(t)))
     return t
 
 
@@ -514,7 +568,7 @@ def mgn_edge_gather_out(nf, ef, src, dst, w1, b1, w2, b2, w3, b3, gamma, beta, o
     _opt("gamma", gamma, (128,))
     _opt("beta", beta, (128,))
     _check_input("out", out, (E, 128))
-    with torch.cuda.device(ef.device):
+    with _on(ef):
         _check(lib.gp_mgn_edge_gather_out(E, N, _ptr(nf), _ptr(ef), _ptr(src), _ptr(dst), src.element_size(),
                                           _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(w3), _ptr(b3), _ptr(gamma),
                                           _ptr(beta), float(eps), _ptr(out), _stream(ef)))
@@ -543,7 +597,7 @@ def gemm_out(x, w, b=None, r=None, act="none", out=None):
     if out is None:
         out = torch.empty((M, N), dtype=dt, device=x.device)
     _check_input("out", out, (M, N), dt)
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_gemm_dtype_out(M, N, K, _ptr(x), _ptr(w), _ptr(b), _ptr(r), ACTS.get(act, act), _ptr(out),
                                      _DTYPES[dt], _stream(x)))
     return out
@@ -572,11 +626,9 @@ def bert_ffn_out(x, w1, b1, w2, b2, ga, be, out, eps=1e-5, act="relu", impl="fus
     _opt("ga", ga, (H,), dt)
     _opt("be", be, (H,), dt)
     _check_input("out", out, (M, H), dt)
-    devs = {t.device for t in (x, w1, b1, w2, b2, ga, be, out) if t is not None}
-    if len(devs) != 1:
-        raise RuntimeError("all tensors must be on the same device")
+    _same_device(x, w1, b1, w2, b2, ga, be, out)
     impl_id = _IMPLS.get(impl, impl)
-    with torch.cuda.device(x.device):
+    with _on(x):
         if impl_id == IMPL_FUSED:
             _check(lib.gp_bert_ffn_dtype_out(M, H, FF, _ptr(x), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(ga),
                                              _ptr(be), float(eps), ACTS.get(act, act), _ptr(out), _DTYPES[dt],
@@ -592,19 +644,13 @@ def bert_ffn_out(x, w1, b1, w2, b2, ga, be, out, eps=1e-5, act="relu", impl="fus
 
 def bert_ffn(x, w1, b1, w2, b2, ga, be, eps=1e-5, act="relu", impl="fused"):
     """Allocating form (bert_ffn_pl_ext.cu:59-72)."""
-    out = torch.zeros_like(x)
+    out = torch.empty_like(x)
     return bert_ffn_out(x, w1, b1, w2, b2, ga, be, out, eps=eps, act=act, impl=impl)
 
 
 # ---------------------------------------------------------------------------
 # Dense MLP chains: DLRM and NeRF
 # ---------------------------------------------------------------------------
-
-def _same_device(*ts):
-    devs = {t.device for t in ts if t is not None}
-    if len(devs) != 1:
-        raise RuntimeError("all tensors must be on the same device")
-
 
 def mlp_out(x, ws, bs, acts, out=None):
     """DlrmMlp-style chain (common/mlps.py:23-34): layer i = acts[i](h @ ws[i] + bs[i]).
@@ -619,11 +665,14 @@ def mlp_out(x, ws, bs, acts, out=None):
     M, K = x.shape
     widths = [K]
     for i, (w, b) in enumerate(zip(ws, bs)):
-        _check_input(f"w{i + 1}", w, dtype=dt)
-        if w.dim() != 2 or w.shape[0] != widths[-1]:
+        if not _ok(w, None, dt):
+            _check_input(f"w{i + 1}", w, dtype=dt)
+        shp = w.shape
+        if len(shp) != 2 or shp[0] != widths[-1]:
             raise RuntimeError(f"w{i + 1} must be [{widths[-1]}, N]")
-        widths.append(w.shape[1])
-        _opt(f"b{i + 1}", b, (w.shape[1],), dt)
+        widths.append(shp[1])
+        if b is not None and not _ok(b, shp[1:], dt):
+            _check_input(f"b{i + 1}", b, shp[1:], dt)
     if out is None:
         out = torch.empty((M, widths[-1]), dtype=dt, device=x.device)
     _check_input("out", out, (M, widths[-1]), dt)
@@ -633,7 +682,7 @@ def mlp_out(x, ws, bs, acts, out=None):
     wp = (ctypes.c_void_p * n)(*[w.data_ptr() for w in ws])
     bp = (ctypes.c_void_p * n)(*[0 if b is None else b.data_ptr() for b in bs])
     ap = (ctypes.c_int * n)(*[ACTS.get(a, a) for a in acts])
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_mlp_dtype_out(M, n, wa, wp, bp, ap, _ptr(x), _ptr(out), _DTYPES[dt], _stream(x)))
     return out
 
@@ -645,7 +694,7 @@ def dlrm_botmlp_out(x, w1, b1, w2, b2, w3, b3, out):
 
 
 def dlrm_botmlp(x, w1, b1, w2, b2, w3, b3):
-    out = torch.zeros((x.shape[0], w3.shape[1]), dtype=x.dtype, device=x.device)
+    out = torch.empty((x.shape[0], w3.shape[1]), dtype=x.dtype, device=x.device)
     return dlrm_botmlp_out(x, w1, b1, w2, b2, w3, b3, out)
 
 
@@ -657,7 +706,7 @@ def dlrm_topmlp_out(x, w1, b1, w2, b2, w3, b3, w4, b4, w5, b5, out, act5="relu")
 
 
 def dlrm_topmlp(x, w1, b1, w2, b2, w3, b3, w4, b4, w5, b5, act5="relu"):
-    out = torch.zeros((x.shape[0], w5.shape[1]), dtype=x.dtype, device=x.device)
+    out = torch.empty((x.shape[0], w5.shape[1]), dtype=x.dtype, device=x.device)
     return dlrm_topmlp_out(x, w1, b1, w2, b2, w3, b3, w4, b4, w5, b5, out, act5=act5)
 
 
@@ -679,15 +728,13 @@ def nerf_full_out(x, d, *wb_and_outs, rgb_act="none"):
     Na, Nrgb = ws[8].shape[1], ws[11].shape[1]
     shapes = [(Kx, 256)] + [(256, 256)] * 4 + [(256 + Kx, 256), (256, 256), (256, 256), (256, Na), (256, 256),
                                                 (256 + Kd, 128), (128, Nrgb)]
-    for i, (w, b, shp) in enumerate(zip(ws, bs, shapes)):
-        _check_input(f"w{i + 1}", w, shp, dt)
-        _opt(f"b{i + 1}", b, (shp[1],), dt)
+    _check_layers(ws, bs, shapes, dt)
     _check_input("out_r", out_r, (M, Na), dt)
     _check_input("out_rgb", out_rgb, (M, Nrgb), dt)
     _same_device(x, d, out_r, out_rgb, *ws, *bs)
     wp = (ctypes.c_void_p * 12)(*[w.data_ptr() for w in ws])
     bp = (ctypes.c_void_p * 12)(*[0 if b is None else b.data_ptr() for b in bs])
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_nerf_full_dtype_out(M, Kx, Kd, Na, Nrgb, _ptr(x), _ptr(d), wp, bp, ACTS.get(rgb_act, rgb_act),
                                           _ptr(out_r), _ptr(out_rgb), _DTYPES[dt], _stream(x)))
     return out_r, out_rgb
@@ -720,7 +767,7 @@ def bert_addln_ffn_out(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, 
     _check_input("out", out, (M, H), dt)
     _same_device(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, out)
     impl_id = _IMPLS.get(impl, impl)
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_bert_addln_ffn_dtype_out(M, H, FF, _ptr(attn_out), _ptr(x), _ptr(w0), _ptr(b0), _ptr(w1),
                                                _ptr(b1), _ptr(w2), _ptr(b2), _ptr(ga0), _ptr(be0), _ptr(ga2),
                                                _ptr(be2), float(eps), ACTS.get(act, act), _ptr(out), int(impl_id),
@@ -731,7 +778,7 @@ def bert_addln_ffn_out(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, 
 def bert_addln_ffn(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, eps=1e-5, act="relu", impl="fused"):
     """Allocating form (bert_addln_ffn_pl_ext.cu:61-76, which passes be0 for be2 -- not
     reproduced: ga2 / be2 are used as given)."""
-    out = torch.zeros_like(x)
+    out = torch.empty_like(x)
     return bert_addln_ffn_out(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, out, eps=eps, act=act,
                               impl=impl)
 
@@ -753,15 +800,13 @@ def nerf_a_out(x, *wb_and_out, impl="fused"):
         raise RuntimeError("x must be 2-D [M, Kx]")
     M, Kx = x.shape
     shapes = [(Kx, 256)] + [(256, 256)] * 4 + [(256 + Kx, 256), (256, 256), (256, 256)]
-    for i, (w, b, shp) in enumerate(zip(ws, bs, shapes)):
-        _check_input(f"w{i + 1}", w, shp, dt)
-        _opt(f"b{i + 1}", b, (256,), dt)
+    _check_layers(ws, bs, shapes, dt)
     _check_input("out", out, (M, 256), dt)
     _same_device(x, out, *ws, *bs)
     wp = (ctypes.c_void_p * 8)(*[w.data_ptr() for w in ws])
     bp = (ctypes.c_void_p * 8)(*[0 if b is None else b.data_ptr() for b in bs])
     impl_id = _IMPLS.get(impl, impl)
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_nerf_a_dtype_out(M, Kx, _ptr(x), wp, bp, _ptr(out), int(impl_id), _DTYPES[dt], _stream(x)))
     return out
 
@@ -770,7 +815,7 @@ def nerf_a(x, *wb, impl="fused"):
     """Allocating form: returns a new [M, 256] tensor (nerf_a_pl_ext.cu:79-110)."""
     if len(wb) != 16:
         raise RuntimeError("expected w1, b1, ..., w8, b8")
-    out = torch.zeros((x.shape[0], 256), dtype=x.dtype, device=x.device)
+    out = torch.empty((x.shape[0], 256), dtype=x.dtype, device=x.device)
     return nerf_a_out(x, *wb, out, impl=impl)
 
 
@@ -790,7 +835,7 @@ def nerf_full_out_noalloc(x, d, *wb_and_outs, rgb_act="none"):
     _same_device(x, d, out_r, out_rgb, *ws, *bs)
     wp = (ctypes.c_void_p * 12)(*[w.data_ptr() for w in ws])
     bp = (ctypes.c_void_p * 12)(*[0 if b is None else b.data_ptr() for b in bs])
-    with torch.cuda.device(x.device):
+    with _on(x):
         _check(lib.gp_nerf_full_out_noalloc(M, Kx, d.shape[1], out_r.shape[1], out_rgb.shape[1], _ptr(x), _ptr(d), wp,
                                             bp, ACTS.get(rgb_act, rgb_act), _ptr(out_r), _ptr(out_rgb), _stream(x)))
     return out_r, out_rgb
@@ -800,6 +845,6 @@ def nerf_full(x, d, *wb, rgb_act="none"):
     """Allocating form: returns (out_r, out_rgb) (nerf_full_pl_ext.cu:99-126)."""
     if len(wb) != 24:
         raise RuntimeError("expected w1, b1, ..., w12, b12")
-    out_r = torch.zeros((x.shape[0], wb[16].shape[1]), dtype=x.dtype, device=x.device)
-    out_rgb = torch.zeros((x.shape[0], wb[22].shape[1]), dtype=x.dtype, device=x.device)
+    out_r = torch.empty((x.shape[0], wb[16].shape[1]), dtype=x.dtype, device=x.device)
+    out_rgb = torch.empty((x.shape[0], wb[22].shape[1]), dtype=x.dtype, device=x.device)
     return nerf_full_out(x, d, *wb, out_r, out_rgb, rgb_act=rgb_act)
