@@ -37,9 +37,9 @@ HIP_FLAGS = [
 # accumulators in AGPRs instead.
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 
-SOURCES = ["mgn_fused.hip", "mgn_pipelined.hip", "stages.hip", "gemm.hip", "gemm_tile.hip", "nerf_fused.hip", "dlrm_fused.hip", "status.hip",
+SOURCES = ["mgn_fused.hip", "mgn_pipelined.hip", "stages.hip", "gemm.hip", "gemm_tile.hip", "ffn_fused.hip", "nerf_fused.hip", "dlrm_fused.hip", "status.hip",
            "bert_addln_pipelined.hip", "bert_ffn_pipelined.hip", "nerf_a_pipelined.hip", "probe.hip", "synth.hip", "capi.cpp", "ffn.cpp", "mlp.cpp", "arena.cpp"]
-SOURCE_FLAGS = {"gemm.hip": [], "nerf_fused.hip": [], "dlrm_fused.hip": []}
+SOURCE_FLAGS = {"gemm.hip": [], "ffn_fused.hip": [], "nerf_fused.hip": [], "dlrm_fused.hip": []}
 
 
 def _run(cmd, verbose):

@@ -882,9 +882,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
   h8 b4 = {}, ones = {};
   b4[0] = bias[64 * wave + lane];
   ones[0] = __builtin_bit_cast(half_t, lane < 32 ? E::kOne : (unsigned short)0);
-  if (threadIdx.x < H2) w5[threadIdx.x] = head[threadIdx.x];
-  const float b5 = head[H2];
   static_for(std::make_integer_sequence<int, PF>{}, [&](auto j) { fetch(j, rp); });
+  const float b5 = head[H2];
+  if (threadIdx.x < H2) w5[threadIdx.x] = head[threadIdx.x];  // (in flight with the first weights)
 
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const int64_t r0 = (int64_t)t * TR;

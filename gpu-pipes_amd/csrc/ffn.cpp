@@ -195,6 +195,15 @@ int gp_bert_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* x, const
   if ((rc = current_device_info(&dev, &ncu))) return rc;
   hipStream_t s = (hipStream_t)stream;
 
+  if (ffn_fused_supported(H, FF)) {
+    void* pack = nullptr;
+    if ((rc = workspace_acquire(dev, s, ffn_fused_workspace(), &pack))) return rc;
+    const BertAddlnArgs a{M, H, FF, x, nullptr, nullptr, nullptr, w1, b1, w2, b2, nullptr, nullptr, gamma, beta, eps,
+                          act, out};
+    const hipError_t e = ffn_fused_launch(a, pack, ncu, s, dtype);
+    return e == hipSuccess ? GP_OK : fail_hip(e, "FFN fused kernel launch");
+  }
+
   // Workspace: w1^T [FF][H], w2^T [H][FF] (unless the GEMMs read w1 and w2
   // in place), then one chunk of activations [CH][FF] and, when the
   // LayerNorm is a launch of its own, of pre-LayerNorm rows [CH][H].
@@ -312,6 +321,14 @@ int gp_bert_addln_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* at
   if (impl == GP_IMPL_PIPELINED) {
     const BertAddlnArgs a{M, H, FF, attn, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, eps, act, out};
     return bert_addln_pipelined_run(a, dev, ncu, s);
+  }
+
+  if (ffn_fused_supported(H, FF)) {
+    void* pack = nullptr;
+    if ((rc = workspace_acquire(dev, s, ffn_fused_workspace(), &pack))) return rc;
+    const BertAddlnArgs a{M, H, FF, attn, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, eps, act, out};
+    const hipError_t e = ffn_fused_launch(a, pack, ncu, s, dtype);
+    return e == hipSuccess ? GP_OK : fail_hip(e, "bert_addln_ffn fused kernel launch");
   }
 
   // Chain: per row chunk, GEMM0 (+ b0 + x), LN0, GEMM1 (+ b1, act), GEMM2 (+ b2 + h0), LN2.

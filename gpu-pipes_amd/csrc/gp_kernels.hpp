@@ -76,6 +76,15 @@ struct BertFfnArgs {
   void* out;
 };
 
+// Either FFN block at the apps' width (H = 128, FF = 512) as one kernel
+// (ffn_fused.hip), any row count: the add + LayerNorm + FFN block, or with w0
+// null the FFN block (attn = x; ga2 / be2 its affine).  All pointers 16-byte
+// aligned; the workspace (ffn_fused_workspace() bytes) receives the packed
+// weights.
+inline bool ffn_fused_supported(int64_t H, int64_t FF) { return H == 128 && FF == 512; }
+size_t ffn_fused_workspace();
+hipError_t ffn_fused_launch(const BertAddlnArgs& a, void* ws, int num_cus, hipStream_t stream, int dtype);
+
 // NerfA of apps/nerf_a (x [M,Kx] -> out [M,256]): five Linear + ReLU layers,
 // the skip concatenation [h | x], three more Linear + ReLU layers.  w[0] is
 // [Kx,256], w[5] [256+Kx,256], the rest [256,256]; biases may be null.

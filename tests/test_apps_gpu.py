@@ -230,3 +230,54 @@ def test_nerf_a_rejects(cuda):
     with pytest.raises(gpipes.GpipesError) as ei:
         nerf_a_gpu(x, ws, bs, "pipelined")
     assert ei.value.code == -2  # Kx must be a multiple of 8 for the pipelined layout
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("act", ["none", "relu", "gelu_tanh", "sigmoid"])
+def test_ffn_fused_matches_chain(cuda, act, dtype):
+    """The one-kernel FFN blocks (H 128, FF 512) against the same block as GEMM and
+    LayerNorm calls: the pre-LayerNorm rows are the same 16-bit values, so outputs
+    agree but for the summation order of the statistics -- every element to one
+    rounding step (plus 2^-18 where the affine cancels), 99% of them bit for bit.
+    Row counts around the 32-row tile and two tiles per CU; biases and affines
+    present and absent; in place."""
+    H, FF = 128, 512
+    g = torch.Generator(device=cuda).manual_seed(3)
+
+    def rnd(*s, k=1.0):
+        return (torch.randn(s, generator=g, device=cuda) * k).to(dtype)
+
+    w0, w1, w2 = rnd(H, H, k=H ** -0.5), rnd(H, FF, k=H ** -0.5), rnd(FF, H, k=FF ** -0.5)
+    full = [rnd(H), rnd(FF), rnd(H), 1 + rnd(H, k=0.2), rnd(H, k=0.2), 1 + rnd(H, k=0.2), rnd(H, k=0.2)]
+    step = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
+
+    def norm(v, ga, be):  # two-pass fp32 LayerNorm of 16-bit rows
+        return torch.nn.functional.layer_norm(v.float(), (H,), None if ga is None else ga.float(),
+                                              None if be is None else be.float(), 1e-5).to(dtype)
+
+    def close(got, want):
+        a, b = got.float(), want.float()
+        tol = torch.maximum(a.abs(), b.abs()) * step + (2.0 ** -18 if dtype == torch.float16 else 2.0 ** -14)
+        assert bool(((a - b).abs() <= tol).all()), (a - b).abs().max().item()
+        assert (got.view(torch.int16) == want.view(torch.int16)).float().mean().item() >= 0.99
+
+    for M in (1, 31, 33, 64, 1000, 16384, 16385, 40001):
+        x, attn = rnd(M, H), rnd(M, H)
+        b0, b1, b2, ga0, be0, ga2, be2 = full if M % 2 else [None] * 7
+        ffn = lambda v: norm(gpipes.gemm_out(gpipes.gemm_out(v, w1, b1, act=act), w2, b2, r=v), ga2, be2)  # noqa: E731
+        y = gpipes.bert_ffn(x, w1, b1, w2, b2, ga2, be2, act=act)
+        close(y, ffn(x))
+        # the second block from its own first LayerNorm's rows
+        z = gpipes.bert_addln_ffn(attn, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, act=act)
+        h0 = norm(gpipes.gemm_out(attn, w0, b0, r=x), ga0, be0)
+        want = ffn(h0)
+        rows = torch.nonzero((z - want).abs().amax(1) > 0.1)  # a flipped rounding of h0 moves its row a little
+        assert rows.numel() == 0
+        rel = (z.float() - want.float()).norm() / want.float().norm()
+        assert rel <= step, rel.item()
+        v = x.clone()
+        gpipes.bert_ffn_out(v, w1, b1, w2, b2, ga2, be2, v, act=act)
+        assert torch.equal(v.view(torch.int16), y.view(torch.int16))
+        v = attn.clone()
+        gpipes.bert_addln_ffn_out(v, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, v, act=act)
+        assert torch.equal(v.view(torch.int16), z.view(torch.int16))
