@@ -150,19 +150,12 @@ int gp_gemm_dtype_out(int64_t M, int64_t N, int64_t K, const void* x, const void
   int dev = 0, ncu = 0;
   if ((rc = current_device_info(&dev, &ncu))) return rc;
   hipStream_t s = (hipStream_t)stream;
-  if (weights_in_place(2.0 * M * N * K)) {
-    GemmArgs g = gemm_w(M, N, K, x, w, b, r, act, out);
-    g.dtype = dtype;
-    const hipError_t e = gemm_launch(g, ncu, s);
-    return e == hipSuccess ? GP_OK : fail_hip(e, "gemm launch");
-  }
-  void* ws = nullptr;
-  if ((rc = workspace_acquire(dev, s, (size_t)N * K * 2, &ws))) return rc;
-  hipError_t e = transpose_launch(w, ws, K, N, s);
-  if (e != hipSuccess) return fail_hip(e, "transpose launch");
-  GemmArgs g{M, N, K, x, ws, b, r, act, out};
+  // (Calls of this much work have never been capturable: they used the
+  // workspace when the weights were still copied.)
+  if (2.0 * M * N * K >= 8e10 && (rc = refuse_capture(s))) return rc;
+  GemmArgs g = gemm_w(M, N, K, x, w, b, r, act, out);
   g.dtype = dtype;
-  e = gemm_launch(g, ncu, s);
+  const hipError_t e = gemm_launch(g, ncu, s);
   return e == hipSuccess ? GP_OK : fail_hip(e, "gemm launch");
 }
 
@@ -204,34 +197,24 @@ int gp_bert_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* x, const
     return e == hipSuccess ? GP_OK : fail_hip(e, "FFN fused kernel launch");
   }
 
-  // Workspace: w1^T [FF][H], w2^T [H][FF] (unless the GEMMs read w1 and w2
-  // in place), then one chunk of activations [CH][FF] and, when the
-  // LayerNorm is a launch of its own, of pre-LayerNorm rows [CH][H].
-  const bool inplace = weights_in_place(4.0 * M * H * FF);
+  // Workspace: one chunk of activations [CH][FF] and, when the LayerNorm is a
+  // launch of its own, of pre-LayerNorm rows [CH][H].
   const int64_t lnch = ln_chunk_rows(H, FF, ncu);
   const bool fuse_ln = lnch > 0;
   if (!fuse_ln && dtype != GP_DTYPE_F16)
     return fail(GP_ERR_SHAPE, "bf16 needs the LayerNorm in the GEMM epilogue, which this device's %d CUs cannot hold", ncu);
   const int64_t chmax = fuse_ln ? lnch : ffn_chunk_rows(FF + H);
   const int64_t CH = M < chmax ? M : chmax;
-  const size_t o_w2t = inplace ? 0 : round_up((size_t)FF * H * 2);
-  const size_t o_act = o_w2t + (inplace ? 0 : round_up((size_t)FF * H * 2));
-  const size_t o_y = o_act + round_up((size_t)CH * FF * 2);
+  const size_t o_y = round_up((size_t)CH * FF * 2);
   const size_t total = o_y + (fuse_ln ? 0 : round_up((size_t)CH * H * 2));
   char* ws = nullptr;
   if ((rc = workspace_acquire(dev, s, total, (void**)&ws))) return rc;
-  void *w1t = ws, *w2t = ws + o_w2t, *hbuf = ws + o_act, *ybuf = ws + o_y;
+  void *hbuf = ws, *ybuf = ws + o_y;
 
   hipError_t e = hipSuccess;
-  if (!inplace) {
-    const PrepSpec ps[2] = {{w1, w1t, nullptr, nullptr, H, FF, H, FF}, {w2, w2t, nullptr, nullptr, FF, H, FF, H}};
-    e = prep_launch(ps, 2, s);
-    if (e != hipSuccess) return fail_hip(e, "transpose launch");
-  }
-  // layer GEMM arguments: the weights in place or their transposed copies
-  auto g = [&](int64_t rows, int64_t N, int64_t K, const void* a, const void* w, const void* wt, const void* b,
-               const void* r, int ac, void* c) {
-    GemmArgs ga = inplace ? gemm_w(rows, N, K, a, w, b, r, ac, c) : GemmArgs{rows, N, K, a, wt, b, r, ac, c};
+  auto g = [&](int64_t rows, int64_t N, int64_t K, const void* a, const void* w, const void* b, const void* r, int ac,
+               void* c) {
+    GemmArgs ga = gemm_w(rows, N, K, a, w, b, r, ac, c);
     ga.dtype = dtype;
     return ga;
   };
@@ -241,15 +224,15 @@ int gp_bert_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* x, const
     const int64_t rows = M - r0 < CH ? M - r0 : CH;
     const void* xc = at_row(x, r0, H);
     char* const oc = (char*)out + r0 * H * 2;
-    e = gemm_launch(g(rows, FF, H, xc, w1, w1t, b1, nullptr, act, hbuf), ncu, s);
+    e = gemm_launch(g(rows, FF, H, xc, w1, b1, nullptr, act, hbuf), ncu, s);
     if (e != hipSuccess) return fail_hip(e, "FFN GEMM1 launch");
     if (fuse_ln) {
       // GEMM2 + bias + residual + LayerNorm
-      e = lne.launch(g(rows, H, FF, hbuf, w2, w2t, b2, xc, GP_ACT_NONE, oc), gamma, beta, eps, ncu, s);
+      e = lne.launch(g(rows, H, FF, hbuf, w2, b2, xc, GP_ACT_NONE, oc), gamma, beta, eps, ncu, s);
       if (e != hipSuccess) return fail_hip(e, "FFN GEMM2 + LayerNorm launch");
       continue;
     }
-    e = gemm_launch(g(rows, H, FF, hbuf, w2, w2t, b2, xc, GP_ACT_NONE, ybuf), ncu, s);
+    e = gemm_launch(g(rows, H, FF, hbuf, w2, b2, xc, GP_ACT_NONE, ybuf), ncu, s);
     if (e != hipSuccess) return fail_hip(e, "FFN GEMM2 launch");
     e = layer_norm_launch(rows, H, ybuf, gamma, beta, eps, oc, ncu, s);
     if (e != hipSuccess) return fail_hip(e, "FFN LayerNorm launch");
@@ -332,37 +315,24 @@ int gp_bert_addln_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* at
   }
 
   // Chain: per row chunk, GEMM0 (+ b0 + x), LN0, GEMM1 (+ b1, act), GEMM2 (+ b2 + h0), LN2.
-  // Workspace: w0^T [H][H], w1^T [FF][H], w2^T [H][FF] (unless the GEMMs
-  // read the weights in place), then for one chunk h0 [CH][H], the
-  // activations [CH][FF] and, when the LayerNorms are launches of their own,
-  // the pre-LayerNorm rows y [CH][H].
-  const bool inplace = weights_in_place(2.0 * M * H * (H + 2.0 * FF));
+  // Workspace, for one chunk: h0 [CH][H], the activations [CH][FF] and, when
+  // the LayerNorms are launches of their own, the pre-LayerNorm rows y [CH][H].
   const int64_t lnch = ln_chunk_rows(H, FF + H, ncu);
   const bool fuse_ln = lnch > 0;
   if (!fuse_ln && dtype != GP_DTYPE_F16)
     return fail(GP_ERR_SHAPE, "bf16 needs the LayerNorm in the GEMM epilogue, which this device's %d CUs cannot hold", ncu);
   const int64_t chmax = fuse_ln ? lnch : ffn_chunk_rows(FF + 2 * H);
   const int64_t CH = M < chmax ? M : chmax;
-  const size_t o_w1t = inplace ? 0 : round_up((size_t)H * H * 2);
-  const size_t o_w2t = o_w1t + (inplace ? 0 : round_up((size_t)FF * H * 2));
-  const size_t o_y = o_w2t + (inplace ? 0 : round_up((size_t)FF * H * 2));
-  const size_t o_h0 = o_y + (fuse_ln ? 0 : round_up((size_t)CH * H * 2));
+  const size_t o_h0 = fuse_ln ? 0 : round_up((size_t)CH * H * 2);
   const size_t o_act = o_h0 + round_up((size_t)CH * H * 2);
   const size_t total = o_act + round_up((size_t)CH * FF * 2);
   char* ws = nullptr;
   if ((rc = workspace_acquire(dev, s, total, (void**)&ws))) return rc;
-  void *w0t = ws, *w1t = ws + o_w1t, *w2t = ws + o_w2t, *ybuf = ws + o_y, *h0 = ws + o_h0, *abuf = ws + o_act;
+  void *ybuf = ws, *h0 = ws + o_h0, *abuf = ws + o_act;
   hipError_t e = hipSuccess;
-  if (!inplace) {
-    const PrepSpec ps[3] = {{w0, w0t, nullptr, nullptr, H, H, H, H},
-                            {w1, w1t, nullptr, nullptr, H, FF, H, FF},
-                            {w2, w2t, nullptr, nullptr, FF, H, FF, H}};
-    e = prep_launch(ps, 3, s);
-    if (e != hipSuccess) return fail_hip(e, "transpose launch");
-  }
-  auto g = [&](int64_t rows, int64_t N, int64_t K, const void* a, const void* w, const void* wt, const void* b,
-               const void* r, int ac, void* c) {
-    GemmArgs ga = inplace ? gemm_w(rows, N, K, a, w, b, r, ac, c) : GemmArgs{rows, N, K, a, wt, b, r, ac, c};
+  auto g = [&](int64_t rows, int64_t N, int64_t K, const void* a, const void* w, const void* b, const void* r, int ac,
+               void* c) {
+    GemmArgs ga = gemm_w(rows, N, K, a, w, b, r, ac, c);
     ga.dtype = dtype;
     return ga;
   };
@@ -373,18 +343,18 @@ int gp_bert_addln_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* at
     if (fuse_ln) {
       // GEMM0 + b0 + x + LN0, GEMM1 + b1 + act, GEMM2 + b2 + h0 + LN2
       char* const oc = (char*)out + r0 * H * 2;
-      e = lne.launch(g(rows, H, H, at_row(attn, r0, H), w0, w0t, b0, at_row(x, r0, H), GP_ACT_NONE, h0), ga0, be0, eps,
+      e = lne.launch(g(rows, H, H, at_row(attn, r0, H), w0, b0, at_row(x, r0, H), GP_ACT_NONE, h0), ga0, be0, eps,
                      ncu, s);
-      if (e == hipSuccess) e = gemm_launch(g(rows, FF, H, h0, w1, w1t, b1, nullptr, act, abuf), ncu, s);
+      if (e == hipSuccess) e = gemm_launch(g(rows, FF, H, h0, w1, b1, nullptr, act, abuf), ncu, s);
       if (e == hipSuccess)
-        e = lne.launch(g(rows, H, FF, abuf, w2, w2t, b2, h0, GP_ACT_NONE, oc), ga2, be2, eps, ncu, s);
+        e = lne.launch(g(rows, H, FF, abuf, w2, b2, h0, GP_ACT_NONE, oc), ga2, be2, eps, ncu, s);
       if (e != hipSuccess) return fail_hip(e, "bert_addln_ffn launch");
       continue;
     }
-    e = gemm_launch(g(rows, H, H, at_row(attn, r0, H), w0, w0t, b0, at_row(x, r0, H), GP_ACT_NONE, ybuf), ncu, s);
+    e = gemm_launch(g(rows, H, H, at_row(attn, r0, H), w0, b0, at_row(x, r0, H), GP_ACT_NONE, ybuf), ncu, s);
     if (e == hipSuccess) e = layer_norm_launch(rows, H, ybuf, ga0, be0, eps, h0, ncu, s);
-    if (e == hipSuccess) e = gemm_launch(g(rows, FF, H, h0, w1, w1t, b1, nullptr, act, abuf), ncu, s);
-    if (e == hipSuccess) e = gemm_launch(g(rows, H, FF, abuf, w2, w2t, b2, h0, GP_ACT_NONE, ybuf), ncu, s);
+    if (e == hipSuccess) e = gemm_launch(g(rows, FF, H, h0, w1, b1, nullptr, act, abuf), ncu, s);
+    if (e == hipSuccess) e = gemm_launch(g(rows, H, FF, abuf, w2, b2, h0, GP_ACT_NONE, ybuf), ncu, s);
     if (e == hipSuccess) e = layer_norm_launch(rows, H, ybuf, ga2, be2, eps, (char*)out + r0 * H * 2, ncu, s);
     if (e != hipSuccess) return fail_hip(e, "bert_addln_ffn launch");
   }

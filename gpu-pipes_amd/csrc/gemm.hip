@@ -11,11 +11,10 @@
 // one streaming kernel over output tiles with its epilogue fused.
 //
 // Kernel design.
-//  * B is consumed transposed (Bt[N][K], from prep_kernel),
-//    so both MFMA operands are rows of consecutive k -- or, for calls small
-//    enough that the transpose launch would cost more than it saves, in its
-//    own [K][N] layout, its fragments read with the transposing LDS read
-//    (the BROW kernels).  The product is computed transposed,
+//  * B is consumed in its own [K][N] layout, its fragments read with the
+//    transposing LDS read (the BROW kernels) -- or, where its width or alignment
+//    does not allow that, transposed and padded (Bt[N][K], from prep_kernel), so
+//    that both MFMA operands are rows of consecutive k.  The product is computed transposed,
 //    C^T = Bt A^T, with v_mfma_f32_32x32x16_f16: the MFMA A operand is a
 //    32-feature block of Bt, the MFMA B operand a 32-row block of A, and each
 //    accumulator lane ends up holding 4 consecutive features of one row.
@@ -755,12 +754,9 @@ template <typename E>
 static hipError_t launch_typed(const GemmArgs& a, Args& g, bool brow, int num_cus, hipStream_t s) {
   if (a.ln) {
     if (a.N == 128 && (a.M + Narrow::BM - 1) / Narrow::BM < num_cus)
-      return brow ? launch<Short, ACT_NONE, true, true, 1, E>(g, num_cus, s)
-                  : launch<Short, ACT_NONE, true, false, 1, E>(g, num_cus, s);
-    if (a.N == 128) return brow ? launch<Narrow, ACT_NONE, true, true, 1, E>(g, num_cus, s)
-                                : launch<Narrow, ACT_NONE, true, false, 1, E>(g, num_cus, s);
-    return brow ? launch<Wide, ACT_NONE, true, true, 2, E>(g, num_cus, s)
-                : launch<Wide, ACT_NONE, true, false, 2, E>(g, num_cus, s);
+      return launch<Short, ACT_NONE, true, true, 1, E>(g, num_cus, s);
+    if (a.N == 128) return launch<Narrow, ACT_NONE, true, true, 1, E>(g, num_cus, s);
+    return launch<Wide, ACT_NONE, true, true, 2, E>(g, num_cus, s);
   }
   if (a.N % Wide::BN == 0) return brow ? dispatch<Wide, true, E>(g, a.act, num_cus, s) : dispatch<Wide, false, E>(g, a.act, num_cus, s);
   return brow ? dispatch<Narrow, true, E>(g, a.act, num_cus, s) : dispatch<Narrow, false, E>(g, a.act, num_cus, s);
@@ -772,9 +768,9 @@ static hipError_t launch_typed(const GemmArgs& a, Args& g, bool brow, int num_cu
 // 65,536, N 128 .. 4096, K 128 .. 4096 (fp16, weights in place, one kernel at
 // a time); within 15% of nearly all and with the fastest kernel of the three
 // on every one of them, e.g. 256-row / 128 x 128 / 64 x 64 tiles:
-//   509 x 1024 x 4096    82 / 34 / 16 us     2048 x 1024 x 1024   26 / 13 / 10
-//   4096 x 1024 x 4096   89 / 41 / 66        8192 x 1024 x 4096   94 / 79 / 141
-//   4096 x 4096 x 1024   38 / 59 / 84        16384 x 1024 x 1024  37 / 50 / 56
+//   509 x 1024 x 4096    83 / 33 / 16 us     2048 x 1024 x 1024   27 / 12 / 10
+//   4096 x 1024 x 4096   87 / 39 / 65        8192 x 1024 x 4096   93 / 73 / 139
+//   4096 x 4096 x 1024   38 / 48 / 84        16384 x 1024 x 1024  37 / 41 / 56
 struct TileCost {
   double best;
   int size;  // 0: the persistent 256-row kernels; 64, 128: gemm_tile.hip
@@ -787,7 +783,8 @@ static TileCost tile_cost(int64_t M, int64_t N, int64_t K, int num_cus) {
   const bool wide = N % Wide::BN == 0;
   const double t256 = tiles(256, wide ? 256 : 128), t128 = tiles(128, 128), t64 = tiles(64, 64);
   const double c256 = 5.0 + rounds(t256, 1) * (slabs * (wide ? 1.0 : 0.55) * (1.15 + 0.75 * load(t256)) + 3.0);
-  const double c128 = 2.5 + rounds(t128, 1) * (slabs * (0.45 + 0.12 * load(t128)) + 3.0);
+  const double c128 =
+      2.5 + rounds(t128, 2) * (t128 > num_cus ? slabs * 1.1 + 4.0 : slabs * (0.45 + 0.1 * load(t128)) + 1.5);
   const double c64 = 3.0 + rounds(t64, 2) * (slabs * (t64 > num_cus ? 0.42 : 0.21) + 1.2);
   if (c256 <= c128 && c256 <= c64) return {c256, 0};
   return c128 <= c64 ? TileCost{c128, 128} : TileCost{c64, 64};
@@ -836,8 +833,9 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t s) {
          (const half_t*)a.gamma, (const half_t*)a.beta, a.eps, nullptr, nullptr, QueueCtx{}, 0};
   if (a.dtype != GP_DTYPE_F16 && a.dtype != GP_DTYPE_BF16) return hipErrorInvalidValue;
   if (a.ln) {
-    // N = 128 (rows within a wave) or 256 .. 1024 in whole 256-feature tiles.
-    if (a.act != ACT_NONE || a.N > 1024 || (a.N != 128 && a.N % Wide::BN) || ((uintptr_t)a.gamma | (uintptr_t)a.beta) % 8)
+    // N = 128 (rows within a wave) or 256 .. 1024 in whole 256-feature tiles;
+    // the weights in place.
+    if (!brow || a.act != ACT_NONE || a.N > 1024 || (a.N != 128 && a.N % Wide::BN) || ((uintptr_t)a.gamma | (uintptr_t)a.beta) % 8)
       return hipErrorInvalidValue;
     if (a.N != 128) {
       if (!a.ln_ws || !a.status || a.epoch == 0 || a.M > gemm_ln_max_rows(a.N, num_cus)) return hipErrorInvalidValue;
@@ -904,15 +902,6 @@ hipError_t gemv1_launch(int64_t M, int64_t K, const void* a, int64_t lda, const 
     hipLaunchKernelGGL(gemm::gemv1_kernel<F16>, dim3((unsigned)grid), dim3(256), 0, s, (const half_t*)a,
                        (int)lda, M, (int)K, (const half_t*)w, (const half_t*)b, act, (half_t*)out);
   return hipGetLastError();
-}
-
-hipError_t transpose_launch(const void* in, void* out, int64_t K, int64_t N, hipStream_t s, int64_t Kp,
-                            int64_t Np) {
-  if (Kp == 0) Kp = K;
-  if (Np == 0) Np = N;
-  if (Kp % 64 != 0 || Np % 64 != 0 || K > Kp || N > Np) return hipErrorInvalidValue;
-  const PrepSpec one{in, out, nullptr, nullptr, K, N, Kp, Np};
-  return prep_launch(&one, 1, s);
 }
 
 }  // namespace gp

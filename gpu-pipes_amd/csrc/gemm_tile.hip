@@ -13,8 +13,12 @@
 // MFMAs run, and the loop is unrolled over the four ring slots, which leaves
 // about 45 instructions a slab at 64 x 64 (75 with the slot in a register:
 // 0.21 against 0.27 us a slab).  A ring of nine slabs ahead instead of three
-// changed nothing.  Two 64 x 64 workgroups share a CU (64 KiB each), one 128 x
-// 128 has it alone.  Measured, 509 x 1024 x 4096 (fp16): 82 us on the
+// changed nothing.  Two workgroups share a CU (64 KiB of LDS each), one's waits
+// under the other's MFMAs: at 128 x 128 that takes slabs of 32 k, and beats one
+// workgroup with slabs of 64 on every shape measured (2048 x 4096 x 1024 27.1
+// -> 23.6 us, 4096 x 1024 x 4096 40.4 -> 39.0).  A 256 x 128 tile of 32-k slabs,
+// two a CU, was behind the persistent kernel where that one fills the chip and
+// behind 128 x 128 where it does not.  Measured, 509 x 1024 x 4096 (fp16): 82 us on the
 // persistent kernel's 8 tiles, 16.3 on 128 tiles of 64 x 64; the calls
 // bert_ffn 509 x 1024 x 4096 134 -> 33 us, DLRM bottom + top at 2,048 rows 118
 // -> 69 us.
@@ -26,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "../../include/gpipes.h"
 #include "gemm_common.hpp"
@@ -37,10 +42,17 @@ namespace tile {
 constexpr int NW = 4;  // waves per workgroup
 constexpr int NT = NW * kWave;
 
-template <int NB, int NS_, int OCC_>
+template <int... I, class F>
+__device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+template <int NB, int BK_, int NS_, int OCC_>
 struct Cfg {
   static constexpr int NBW = NB, MBW = NB, WN = 2, WM = 2;       // 32-feature / 32-row blocks per wave, waves
   static constexpr int BN = 32 * NBW * WN, BM = 32 * MBW * WM;   // features and rows per tile
+  static constexpr int BK = BK_, KS = BK / 16;                   // k and MFMA steps per slab
+  static constexpr int ROWB = 2 * BK, CPR = ROWB / 16, RPC = 64 / CPR;  // bytes and chunks of a slab row, rows per copy
   static constexpr int NS = NS_;                                 // slabs in the LDS ring
   static constexpr int OCC = OCC_;                               // workgroups per CU
   static constexpr int ABYTES = BM * ROWB, BBYTES = BN * ROWB;   // bytes of a slab's A and B part
@@ -50,8 +62,21 @@ struct Cfg {
   static_assert(NS >= 3 && OCC * NS * STAGE <= 160 * 1024, "LDS");
   static_assert((NS - 1) * (UA + UB) <= 63, "copies in flight exceed the counter field");
 };
-using T64 = Cfg<1, 4, 2>;
-using T128 = Cfg<2, 4, 1>;
+using T64 = Cfg<1, 64, 4, 2>;
+using T128 = Cfg<2, 32, 4, 2>;
+
+// Byte offset of 16-byte chunk c of row r in an operand slab of ROWB-byte rows:
+// XOR-swizzled so that 16 consecutive rows read at one chunk cover all of the
+// 16-byte bank groups (128-byte rows: unit_off; 64-byte rows lie four to a
+// 256-byte bank window).
+template <class C>
+__device__ __forceinline__ int row_swz(int r) {
+  return C::ROWB == 128 ? (r >> 1) & 7 : (r >> 2) & 3;
+}
+template <class C>
+__device__ __forceinline__ int row_off(int r, int c) {
+  return r * C::ROWB + ((c ^ row_swz<C>(r)) << 4);
+}
 
 // Chunk swizzle of row r of a weight slab kept in its own [k][feature] layout
 // (16-byte chunks; BN = 64: eight to a row, two rows to a 256-byte bank
@@ -67,6 +92,7 @@ template <class C, int ACT, bool RESID, bool BROW, typename E>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C::OCC, C::OCC))) void tile_kernel(Args p) {
   __shared__ __attribute__((aligned(1024))) char ring[C::NS * C::STAGE];
   constexpr int NS = C::NS, CPS = C::UA + C::UB;  // ring slabs, copies per wave and slab
+  constexpr int BK = C::BK, KS = C::KS, ROWB = C::ROWB, CPR = C::CPR, RPC = C::RPC;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -106,7 +132,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C::OCC, C::O
   // consecutive j are 32 apart, which leaves the swizzle unchanged.  A weight
   // slab in its own layout: 64 rows of BN features, RB rows to a copy.
   const int vrow = RPC * wave + lane / CPR;
-  const int vswz = ((lane % CPR) ^ ((vrow >> 1) & 7)) << 4;
+  const int vswz = ((lane % CPR) ^ row_swz<C>(vrow)) << 4;
   const int voffa = vrow * p.lda * 2 + vswz;
   constexpr int CB = C::BN / 8, RB = 64 / CB;
   const int rq = RB * wave + lane / CB;
@@ -176,8 +202,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C::OCC, C::O
   GP_LDS const char* pb[BROW ? C::NBW : KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
-    pa[ks] = (GP_LDS const char*)ring + unit_off(arow, 2 * ks + lh);
-    if constexpr (!BROW) pb[ks] = (GP_LDS const char*)ring + C::ABYTES + unit_off(frow, 2 * ks + lh);
+    pa[ks] = (GP_LDS const char*)ring + row_off<C>(arow, 2 * ks + lh);
+    if constexpr (!BROW) pb[ks] = (GP_LDS const char*)ring + C::ABYTES + row_off<C>(frow, 2 * ks + lh);
   }
   if constexpr (BROW) {
 #pragma unroll
@@ -213,31 +239,29 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C::OCC, C::O
   wait_vmcnt<(NS - 1) * CPS>();
   lds_barrier();
   load(f[0], 0);
-  // Slab kt, which lives in ring slot S = kt % NS and register set S % 2.
-  static_assert(NS % 2 == 0, "slots and register sets alternate together");
-  auto step = [&](int kt, auto slot) {
-    constexpr int S = decltype(slot)::value, S1 = (S + 1) % NS;
+  // Slab kt, which lives in ring slot kt % NS and register set kt % 2; U is kt
+  // modulo the unrolling, a multiple of both.
+  constexpr int UNROLL = NS % 2 ? 2 * NS : NS;
+  auto step = [&](int kt, auto uc) {
+    constexpr int U = decltype(uc)::value, S = U % NS, S1 = (U + 1) % NS;
     // This wave's copies of slab kt + 1 have landed once at most the NS - 2
     // slabs issued after it are in flight; past the barrier every wave's have,
     // and every wave holds slab kt in registers, so its slot takes slab kt + NS.
     wait_vmcnt<(NS - 2) * CPS>();
     lds_barrier();
-    load(f[S1 % 2], S1);
+    load(f[(U + 1) % 2], S1);
     issue(kt + NS, S);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int nb = 0; nb < C::NBW; ++nb)
 #pragma unroll
-        for (int mb = 0; mb < C::MBW; ++mb) acc[nb][mb] = E::mma(f[S % 2].a[ks][nb], f[S % 2].b[ks][mb], acc[nb][mb]);
+        for (int mb = 0; mb < C::MBW; ++mb) acc[nb][mb] = E::mma(f[U % 2].a[ks][nb], f[U % 2].b[ks][mb], acc[nb][mb]);
   };
-  for (int kt = 0; kt < nslab; kt += NS) {
-    step(kt, std::integral_constant<int, 0>{});
-    if (kt + 1 < nslab) step(kt + 1, std::integral_constant<int, 1>{});
-    if (kt + 2 < nslab) step(kt + 2, std::integral_constant<int, 2>{});
-    if (kt + 3 < nslab) step(kt + 3, std::integral_constant<int, 3>{});
-  }
-  static_assert(NS == 4, "the loop above is unrolled over the slots");
+  for (int kt = 0; kt < nslab; kt += UNROLL)
+    static_for(std::make_integer_sequence<int, UNROLL>{}, [&](auto uc) {
+      if (uc == 0 || kt + uc < nslab) step(kt + uc, uc);
+    });
 
   // Epilogue: lane (lr, lh) holds, in elements 4 g + e of block (nb, mb), row
   // arow + 32 mb and feature n0 + 32 (NBW wn + nb) + 8 g + 4 lh + e.  The

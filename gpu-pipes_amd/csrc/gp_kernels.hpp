@@ -172,27 +172,19 @@ bool gemm_ln_apart(int64_t M, int64_t N, int64_t K, int num_cus);
 // gamma / beta may be null (1 / 0).  In place when out == x.
 hipError_t gemm_ln_rows_launch(int64_t M, int64_t N, const void* x, const void* gamma, const void* beta, float eps,
                                void* out, int dtype, hipStream_t s);
-// Whether a layer chain reads its weights in place instead of from
-// transposed copies.  In place, each weight fragment of the GEMM's k-loop
-// takes two transposing LDS reads instead of one 16-byte read, which slows
-// the loop by about 15% (BERT-large FFN 1.21 -> 1.38 ms); the copies cost one
-// transpose launch per call (5-9 us).  Below kInPlaceMaxFlop of GEMM work
-// (about 80 us) in place comes out ahead: the bert_addln_ffn chain at its
-// app's batch 0.1165 -> 0.1148 ms, nerf_a 0.1788 -> 0.1737 ms.
-constexpr double kInPlaceMaxFlop = 8e10;
-inline bool weights_in_place(double flop) { return flop < kInPlaceMaxFlop; }
-
-// GEMM arguments for W [K, N] read in place (row stride N).
+// GEMM arguments for W [K, N] read in place (row stride N).  Every 16-byte
+// aligned weight of a width that is a multiple of 128 is read this way: two
+// transposing LDS reads a fragment instead of one 16-byte read cost the K loop
+// nothing measurable (16384 x 1024 x 4096 117.9 us either way, 65536 x 1024 x
+// 1024 138.3 from a transposed copy, 140.5 in place), and the copy was a launch
+// of 7 to 14 us per call: BERT-large FFN, 65,536 rows, 1140 -> 1126 us, DLRM
+// bottom + top, 262,144 rows, 1394 -> 1364 us.
 inline GemmArgs gemm_w(int64_t M, int64_t N, int64_t K, const void* x, const void* w, const void* b, const void* r,
                        int act, void* out) {
   GemmArgs g{M, N, K, x, nullptr, b, r, act, out};
   g.w = w;
   return g;
 }
-// out[Np, Kp] = in[K, N]^T, zero-padded (Kp, Np default to K, N); Kp and Np
-// multiples of 64.
-hipError_t transpose_launch(const void* in, void* out, int64_t K, int64_t N, hipStream_t stream, int64_t Kp = 0,
-                            int64_t Np = 0);
 // out[m] = act(a[m, 0:K] . w[0:K] + b[0]) for m < M (a one-output layer); K
 // and lda multiples of 8, a and w 16-byte aligned, b may be null.
 hipError_t gemv1_launch(int64_t M, int64_t K, const void* a, int64_t lda, const void* w, const void* b, int act,

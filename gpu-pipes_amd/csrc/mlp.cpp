@@ -10,8 +10,9 @@
 // here every layer is one launch of the wide GEMM stage (gemm.hip) with its
 // bias and activation fused, over row chunks of 262,144.
 // Narrow and odd widths are handled by padding, never by special kernels:
-//   * weights are transposed into the workspace with zero rows and columns up
-//     to K a multiple of 64 and N a multiple of 128, biases zero-padded to N;
+//   * weights that the GEMM cannot read in place (in_place below) are transposed
+//     into the workspace with zero rows and columns up to K a multiple of 64 and
+//     N a multiple of 128, their biases zero-padded to N;
 //   * an input whose width is not a multiple of 8 (or not 16-byte aligned) is
 //     copied into a padded buffer; other inputs are read in place, and the
 //     GEMM zero-fills the columns past their width;
@@ -68,12 +69,11 @@ struct Prepared {
   int64_t kw = 0;
 };
 
-// A layer of a chain small enough to read its weights in place
-// (weights_in_place) does so when its output width is a multiple of 128 and
-// weights and bias are 16-byte aligned; otherwise they are prepared
+// A layer reads its weights in place when its output width is a multiple of
+// 128 and weights and bias are 16-byte aligned; otherwise they are prepared
 // (transposed, zero-padded) into the workspace by the chain's prep launch.
-bool in_place(bool chain, int64_t N, const void* w, const void* b) {
-  return chain && N % 128 == 0 && aligned16(w) && (!b || aligned16(b));
+bool in_place(int64_t N, const void* w, const void* b) {
+  return N % 128 == 0 && aligned16(w) && (!b || aligned16(b));
 }
 
 
@@ -167,11 +167,8 @@ int run_chain(int64_t M, int nl, const int64_t* widths, const void* const* w, co
   // own.
   std::vector<Prepared> L(nl);
   std::vector<PrepSpec> ps;
-  double flop = 0;
-  for (int i = 0; i < nl; ++i) flop += 2.0 * M * widths[i] * widths[i + 1];
-  const bool chain = weights_in_place(flop);
   for (int i = 0; i < (fused_tail ? tl : nl); ++i) {
-    if (in_place(chain, widths[i + 1], w[i], b[i])) {
+    if (in_place(widths[i + 1], w[i], b[i])) {
       L[i] = {nullptr, b[i], kin[i], np[i], acts[i], w[i], widths[i]};
     } else {
       ps.push_back({w[i], ws + o_wt[i], b[i], ws + o_b[i], widths[i], widths[i + 1], kin[i], np[i]});
@@ -356,11 +353,8 @@ int gp_nerf_full_dtype_out(int64_t M, int64_t Kx, int64_t Kd, int64_t Na, int64_
   Prepared L[12];
   PrepSpec ps[12];
   int nps = 0;
-  double flop = 0;
-  for (int i = 0; i < 12; ++i) flop += 2.0 * M * sh[i].K * sh[i].N;
-  const bool chain = weights_in_place(flop);
   for (int i = 0; i < 12; ++i) {
-    if (in_place(chain, sh[i].N, w[i], b[i])) {
+    if (in_place(sh[i].N, w[i], b[i])) {
       L[i] = {nullptr, b[i], sh[i].Kin, sh[i].Np, sh[i].act, w[i], sh[i].K};
     } else {
       ps[nps++] = {w[i], ws + o_wt[i], b[i], ws + o_b[i], sh[i].K, sh[i].N, sh[i].Kin, sh[i].Np};
@@ -480,11 +474,8 @@ int gp_nerf_a_dtype_out(int64_t M, int64_t Kx, const void* x, const void* const*
   Prepared L[8];
   PrepSpec ps[8];
   int nps = 0;
-  double flop = 0;
-  for (int i = 0; i < 8; ++i) flop += 2.0 * M * kreal[i] * H;
-  const bool chain = weights_in_place(flop);
   for (int i = 0; i < 8; ++i) {
-    if (in_place(chain, H, w[i], b[i])) {
+    if (in_place(H, w[i], b[i])) {
       L[i] = {nullptr, b[i], kin[i], H, GP_ACT_RELU, w[i], kreal[i]};
     } else {
       ps[nps++] = {w[i], ws + o_wt[i], b[i], ws + o_b[i], kreal[i], H, kin[i], H};
