@@ -297,6 +297,12 @@ static int persistent_grid(int64_t M, int num_cus, int per_cu) {
 template <int K, int ACT, bool LN>
 static hipError_t launch_linear(const LinearArgs& a, int num_cus, hipStream_t s) {
   constexpr int lds = gemm_stage_lds<MBLK, K, kLinearBufs>() + kGemmParamLds;
+  // Workgroups per CU: at K = 128 LDS holds two, and one's weight prologue,
+  // epilogue and last partial round run under the other's tiles (50,001 rows
+  // 9.1 -> 8.4 us, with LayerNorm 12.2 -> 10.6; 262,144 rows 29 -> 27.6 and 36 ->
+  // 31.5).  Wider inputs fill it alone.
+  constexpr int kPerCu = K == 128 ? 2 : 1;
+  static_assert(kPerCu * lds <= 160 * 1024, "LDS");
   auto kern = linear_kernel<K, ACT, LN>;
   // The LDS limit is set once per device (not per launch, so that a launch
   // under graph capture makes no other runtime call).
@@ -310,7 +316,7 @@ static hipError_t launch_linear(const LinearArgs& a, int num_cus, hipStream_t s)
     if (e != hipSuccess) return e;
     lds_set[dev].store(true, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kern, dim3(persistent_grid(a.M, num_cus, 1)), dim3(kStageThreads), lds, s, a);
+  hipLaunchKernelGGL(kern, dim3(persistent_grid(a.M, num_cus, kPerCu)), dim3(kStageThreads), lds, s, a);
   return hipGetLastError();
 }
 
