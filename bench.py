@@ -385,7 +385,7 @@ def bench_bert(args):
             "frac": tflops / MFMA_F16_PEAK_TFLOPS, "traffic": None,
             "kernel_ms_avg": avg_ms, "kernel_ms_median": spread(call_ms)["median"],
             "flops_per_launch": flops, "algorithmic_bytes_per_launch": bytes_,
-            "launch": "one gp_bert_ffn_out call (one weight-transpose launch, then per 16384-row chunk: "
+            "launch": "one gp_bert_ffn_out call (per 16384-row chunk: "
                       "GEMM1+bias+GELU, GEMM2+bias+residual+LayerNorm)",
         },
         "spread": spread(call_ms),
@@ -587,11 +587,11 @@ def bench_chain(args):
         data = "synthetic (positional encodings of U(-1,1) points and unit directions, Kaiming-uniform, seed 0)"
         unit = "samples/s"
     launch = {"dlrm": "one step: the bottom MLP as a weight-packing launch plus one fused three-layer kernel "
-                      "over 256-row tiles; the top MLP as one weight-preparation launch, a wide-GEMM launch for "
+                      "over 256-row tiles; the top MLP as a wide-GEMM launch for "
                       "each of its first three layers, then a weight-packing launch plus one fused kernel for "
                       "512 -> 256 -> 1 (the click head)",
               "nerf": "one step: the weight-packing kernel, then the fused 12-layer kernel over 256-row tiles",
-              "bert_addln": "one step: one gp_bert_addln_ffn_out call (fused: weight transposes, then GEMM0 + b0 + x, "
+              "bert_addln": "one step: one gp_bert_addln_ffn_out call (fused: the weight-packing kernel, then one kernel of GEMM0 + b0 + x, "
                             "LN0, GEMM1 + act, GEMM2 + b2 + h0, LN2; pipelined: one queue-chained kernel)",
               "nerf_a": "one step: one gp_nerf_a_out call (fused: the weight-packing kernel, then the NeRF kernel "
                         "stopped after layer 8; pipelined: one queue-chained kernel)",
@@ -770,7 +770,7 @@ def bench_gemm(args):
             "value": flops / (ours * 1e-3) / 1e12, "unit": "TFLOP/s", "n_gpus": 1, "ms_per_step": ours,
             "higher_is_better": True, "dtype": "f16", "data": "synthetic (N(0,1) inputs, N(0,1/K) weights)",
             "config": {"workload": "gemm", "M": M, "K": K, "N": N,
-                       "weights": "in place" if 2.0 * M * N * K < 8e10 else "transposed copy made by the call"},
+                       "weights": "in place"},
             "library": {"name": f"torch {torch.__version__} matmul (hipBLASLt), no epilogue", "ms": lib_ms,
                         "tflops": flops / (lib_ms * 1e-3) / 1e12},
         }), flush=True)
