@@ -232,6 +232,31 @@ def test_gemm_weight_paths_agree(cuda):
                   "gemm transposed-copy path, sampled rows")
 
 
+@pytest.mark.parametrize("M,N,K,act", [
+    (30011, 512, 1024, "relu"),        # 118 x 2 tiles of 256 x 256 on 240 workgroups
+    (14999, 1024, 256, "gelu_tanh"),   # 59 x 4
+    (20011, 384, 1024, "none"),        # 79 x 3 tiles of 256 x 128
+    (32001, 512, 128, "relu"),         # 126 x 2
+    (50001, 512, 128, "gelu_tanh"),    # 196 x 2: more tiles than CUs
+    (100003, 512, 128, "relu"),        # 391 x 2
+    (50001, 1024, 256, "relu"),        # 196 x 4
+])
+def test_gemm_ragged_tile_counts(cuda, M, N, K, act):
+    """Row counts whose tiles are no multiple of the XCDs, up to where one tile
+    size takes over from the other: every row is written once, and as in a call
+    of a few rows (other tiles, the same products in the same order)."""
+    g = torch.Generator(device=cuda).manual_seed(M)
+    x = torch.randn((M, K), generator=g, device=cuda).half()
+    w = (torch.randn((K, N), generator=g, device=cuda) / K ** 0.5).half()
+    b = torch.randn((N,), generator=g, device=cuda).half()
+    y = gpipes.gemm_out(x, w, b, act=act, out=torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda))
+    for r0 in range(0, M, 4096):
+        part = gpipes.gemm_out(x[r0:r0 + 509].contiguous(), w, b, act=act)
+        assert torch.equal(y[r0:r0 + 509].view(torch.int16), part.view(torch.int16)), r0
+    assert not torch.isnan(y).any()
+    assert_parity(f(y[-300:]), oracle.linear(f(x[-300:]), f(w), f(b), ACT_ID[act]), f"gemm M={M} N={N} K={K}")
+
+
 def test_gemm_identity_weight_is_exact(cuda):
     """x . I (+ 0) passes every fp16 value through the fp32 accumulator unchanged."""
     M, K = 700, 256
