@@ -789,9 +789,18 @@ static TileCost tile_cost(int64_t M, int64_t N, int64_t K, int num_cus) {
   auto load = [&](double t) { return t < num_cus ? t / num_cus : 1.0; };
   const bool wide = N % Wide::BN == 0;
   const double t256 = tiles(256, wide ? 256 : 128), t128 = tiles(128, 128), t64 = tiles(64, 64);
-  const double c256 = 5.0 + rounds(t256, 1) * (slabs * (wide ? 1.0 : 0.55) * (1.15 + 0.75 * load(t256)) + 3.0);
+  // Short walks over many rounds: the epilogue is most of a round of the
+  // 256 x 256 tiles, which nothing hides (5.3 us), and tiles that start whenever
+  // one ends do not wait for whole rounds.  256-row / 128 x 128 tiles, per call:
+  // 50,001 x 128 -> 512 GELU 25.2 / 23.8 us, 100,000 x 128 -> 512 40.8 / 35.4,
+  // 50,001 x 256 -> 1024 54.8 / 48.2.  At K = 256 and two rounds the two tie
+  // (50,001 x 256 -> 512 27.1 / 28.4, GELU 31.1 / 30.9).
+  const bool shallow = wide && (K <= 128 || (K <= 256 && rounds(t256, 1) > 2)) && t256 > num_cus;
+  const double c256 =
+      5.0 + rounds(t256, 1) * (slabs * (wide ? 1.0 : 0.55) * (1.15 + 0.75 * load(t256)) + (shallow ? 5.3 : 3.0));
   const double c128 =
-      2.5 + rounds(t128, 2) * (t128 > num_cus ? slabs * 1.1 + 4.0 : slabs * (0.45 + 0.1 * load(t128)) + 1.5);
+      2.5 + (shallow ? t128 / (2.0 * num_cus) : rounds(t128, 2)) *
+                (t128 > num_cus ? slabs * 1.1 + 4.0 : slabs * (0.45 + 0.1 * load(t128)) + 1.5);
   const double c64 = 3.0 + rounds(t64, 2) * (slabs * (t64 > num_cus ? 0.42 : 0.21) + 1.2);
   if (c256 <= c128 && c256 <= c64) return {c256, 0};
   return c128 <= c64 ? TileCost{c128, 128} : TileCost{c64, 64};
