@@ -122,6 +122,45 @@ int64_t ln_chunk_rows(int64_t H, int64_t row_elems, int ncu) {
   return r < 256 ? 0 : (r < c ? r : c);
 }
 
+// The weights of a call's layers, W [K, N] each: read in place, or where
+// gemm_copy_weights says so from a transposed copy in the workspace.  Added in
+// the order of the layers; then base is set and copy() launched once.
+struct Weights {
+  struct Layer {
+    int64_t N, K;
+    const void* w;
+    bool copied;
+    size_t off;  // of the copy
+  };
+  int64_t M, rows;
+  int ncu;
+  Layer L[3];
+  int n = 0;
+  size_t bytes = 0;  // workspace of the copies
+  char* base = nullptr;
+
+  Weights(int64_t M_, int64_t rows_, int ncu_) : M(M_), rows(rows_), ncu(ncu_) {}
+  // ln: the layer ends in a LayerNorm.
+  void add(int64_t N, int64_t K, const void* w, bool ln) {
+    const bool c = gemm_copy_weights(M, rows, N, K, ln, ncu);
+    L[n++] = {N, K, w, c, bytes};
+    if (c) bytes += round_up((size_t)N * K * 2);
+  }
+  hipError_t copy(hipStream_t s) const {
+    PrepSpec ps[3];
+    int m = 0;
+    for (int i = 0; i < n; ++i)
+      if (L[i].copied) ps[m++] = {L[i].w, base + L[i].off, nullptr, nullptr, L[i].K, L[i].N, L[i].K, L[i].N};
+    return m ? prep_launch(ps, m, s) : hipSuccess;
+  }
+  GemmArgs gemm(int i, int64_t M_, const void* x, const void* b, const void* r, int act, void* out, int dtype) const {
+    GemmArgs g{M_, L[i].N, L[i].K, x, L[i].copied ? base + L[i].off : nullptr, b, r, act, out};
+    if (!L[i].copied) g.w = L[i].w;
+    g.dtype = dtype;
+    return g;
+  }
+};
+
 }  // namespace
 }  // namespace gp
 
@@ -150,12 +189,15 @@ int gp_gemm_dtype_out(int64_t M, int64_t N, int64_t K, const void* x, const void
   int dev = 0, ncu = 0;
   if ((rc = current_device_info(&dev, &ncu))) return rc;
   hipStream_t s = (hipStream_t)stream;
+  Weights W(M, M, ncu);
+  W.add(N, K, w, false);
+  if (W.bytes && (rc = workspace_acquire(dev, s, W.bytes, (void**)&W.base))) return rc;
   // (Calls of this much work have never been capturable: they used the
   // workspace when the weights were still copied.)
   if (2.0 * M * N * K >= 8e10 && (rc = refuse_capture(s))) return rc;
-  GemmArgs g = gemm_w(M, N, K, x, w, b, r, act, out);
-  g.dtype = dtype;
-  const hipError_t e = gemm_launch(g, ncu, s);
+  hipError_t e = W.copy(s);
+  if (e != hipSuccess) return fail_hip(e, "transpose launch");
+  e = gemm_launch(W.gemm(0, M, x, b, r, act, out, dtype), ncu, s);
   return e == hipSuccess ? GP_OK : fail_hip(e, "gemm launch");
 }
 
@@ -197,42 +239,38 @@ int gp_bert_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* x, const
     return e == hipSuccess ? GP_OK : fail_hip(e, "FFN fused kernel launch");
   }
 
-  // Workspace: one chunk of activations [CH][FF] and, when the LayerNorm is a
-  // launch of its own, of pre-LayerNorm rows [CH][H].
+  // Workspace: the weights that are copied, one chunk of activations [CH][FF]
+  // and, when the LayerNorm is a launch of its own, of pre-LayerNorm rows [CH][H].
   const int64_t lnch = ln_chunk_rows(H, FF, ncu);
   const bool fuse_ln = lnch > 0;
   if (!fuse_ln && dtype != GP_DTYPE_F16)
     return fail(GP_ERR_SHAPE, "bf16 needs the LayerNorm in the GEMM epilogue, which this device's %d CUs cannot hold", ncu);
   const int64_t chmax = fuse_ln ? lnch : ffn_chunk_rows(FF + H);
   const int64_t CH = M < chmax ? M : chmax;
-  const size_t o_y = round_up((size_t)CH * FF * 2);
+  Weights W(M, CH, ncu);
+  W.add(FF, H, w1, false);
+  W.add(H, FF, w2, true);
+  const size_t o_act = W.bytes, o_y = o_act + round_up((size_t)CH * FF * 2);
   const size_t total = o_y + (fuse_ln ? 0 : round_up((size_t)CH * H * 2));
-  char* ws = nullptr;
-  if ((rc = workspace_acquire(dev, s, total, (void**)&ws))) return rc;
-  void *hbuf = ws, *ybuf = ws + o_y;
-
-  hipError_t e = hipSuccess;
-  auto g = [&](int64_t rows, int64_t N, int64_t K, const void* a, const void* w, const void* b, const void* r, int ac,
-               void* c) {
-    GemmArgs ga = gemm_w(rows, N, K, a, w, b, r, ac, c);
-    ga.dtype = dtype;
-    return ga;
-  };
+  if ((rc = workspace_acquire(dev, s, total, (void**)&W.base))) return rc;
+  void *hbuf = W.base + o_act, *ybuf = W.base + o_y;
+  hipError_t e = W.copy(s);
+  if (e != hipSuccess) return fail_hip(e, "transpose launch");
   LnEpilogue lne;
   if (fuse_ln && (rc = lne.init(dev, s, CH, H, !gemm_ln_apart(CH, H, FF, ncu)))) return rc;
   for (int64_t r0 = 0; r0 < M; r0 += CH) {
     const int64_t rows = M - r0 < CH ? M - r0 : CH;
     const void* xc = at_row(x, r0, H);
     char* const oc = (char*)out + r0 * H * 2;
-    e = gemm_launch(g(rows, FF, H, xc, w1, b1, nullptr, act, hbuf), ncu, s);
+    e = gemm_launch(W.gemm(0, rows, xc, b1, nullptr, act, hbuf, dtype), ncu, s);
     if (e != hipSuccess) return fail_hip(e, "FFN GEMM1 launch");
     if (fuse_ln) {
       // GEMM2 + bias + residual + LayerNorm
-      e = lne.launch(g(rows, H, FF, hbuf, w2, b2, xc, GP_ACT_NONE, oc), gamma, beta, eps, ncu, s);
+      e = lne.launch(W.gemm(1, rows, hbuf, b2, xc, GP_ACT_NONE, oc, dtype), gamma, beta, eps, ncu, s);
       if (e != hipSuccess) return fail_hip(e, "FFN GEMM2 + LayerNorm launch");
       continue;
     }
-    e = gemm_launch(g(rows, H, FF, hbuf, w2, b2, xc, GP_ACT_NONE, ybuf), ncu, s);
+    e = gemm_launch(W.gemm(1, rows, hbuf, b2, xc, GP_ACT_NONE, ybuf, dtype), ncu, s);
     if (e != hipSuccess) return fail_hip(e, "FFN GEMM2 launch");
     e = layer_norm_launch(rows, H, ybuf, gamma, beta, eps, oc, ncu, s);
     if (e != hipSuccess) return fail_hip(e, "FFN LayerNorm launch");
@@ -315,27 +353,26 @@ int gp_bert_addln_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* at
   }
 
   // Chain: per row chunk, GEMM0 (+ b0 + x), LN0, GEMM1 (+ b1, act), GEMM2 (+ b2 + h0), LN2.
-  // Workspace, for one chunk: h0 [CH][H], the activations [CH][FF] and, when
-  // the LayerNorms are launches of their own, the pre-LayerNorm rows y [CH][H].
+  // Workspace: the weights that are copied and, for one chunk, h0 [CH][H], the
+  // activations [CH][FF] and, when the LayerNorms are launches of their own, the
+  // pre-LayerNorm rows y [CH][H].
   const int64_t lnch = ln_chunk_rows(H, FF + H, ncu);
   const bool fuse_ln = lnch > 0;
   if (!fuse_ln && dtype != GP_DTYPE_F16)
     return fail(GP_ERR_SHAPE, "bf16 needs the LayerNorm in the GEMM epilogue, which this device's %d CUs cannot hold", ncu);
   const int64_t chmax = fuse_ln ? lnch : ffn_chunk_rows(FF + 2 * H);
   const int64_t CH = M < chmax ? M : chmax;
-  const size_t o_h0 = fuse_ln ? 0 : round_up((size_t)CH * H * 2);
+  Weights W(M, CH, ncu);
+  W.add(H, H, w0, true);
+  W.add(FF, H, w1, false);
+  W.add(H, FF, w2, true);
+  const size_t o_y = W.bytes, o_h0 = o_y + (fuse_ln ? 0 : round_up((size_t)CH * H * 2));
   const size_t o_act = o_h0 + round_up((size_t)CH * H * 2);
   const size_t total = o_act + round_up((size_t)CH * FF * 2);
-  char* ws = nullptr;
-  if ((rc = workspace_acquire(dev, s, total, (void**)&ws))) return rc;
-  void *ybuf = ws, *h0 = ws + o_h0, *abuf = ws + o_act;
-  hipError_t e = hipSuccess;
-  auto g = [&](int64_t rows, int64_t N, int64_t K, const void* a, const void* w, const void* b, const void* r, int ac,
-               void* c) {
-    GemmArgs ga = gemm_w(rows, N, K, a, w, b, r, ac, c);
-    ga.dtype = dtype;
-    return ga;
-  };
+  if ((rc = workspace_acquire(dev, s, total, (void**)&W.base))) return rc;
+  void *ybuf = W.base + o_y, *h0 = W.base + o_h0, *abuf = W.base + o_act;
+  hipError_t e = W.copy(s);
+  if (e != hipSuccess) return fail_hip(e, "transpose launch");
   LnEpilogue lne;
   if (fuse_ln && (rc = lne.init(dev, s, CH, H, !gemm_ln_apart(CH, H, H, ncu) || !gemm_ln_apart(CH, H, FF, ncu)))) return rc;
   for (int64_t r0 = 0; r0 < M; r0 += CH) {
@@ -343,18 +380,18 @@ int gp_bert_addln_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* at
     if (fuse_ln) {
       // GEMM0 + b0 + x + LN0, GEMM1 + b1 + act, GEMM2 + b2 + h0 + LN2
       char* const oc = (char*)out + r0 * H * 2;
-      e = lne.launch(g(rows, H, H, at_row(attn, r0, H), w0, b0, at_row(x, r0, H), GP_ACT_NONE, h0), ga0, be0, eps,
-                     ncu, s);
-      if (e == hipSuccess) e = gemm_launch(g(rows, FF, H, h0, w1, b1, nullptr, act, abuf), ncu, s);
+      e = lne.launch(W.gemm(0, rows, at_row(attn, r0, H), b0, at_row(x, r0, H), GP_ACT_NONE, h0, dtype), ga0, be0,
+                     eps, ncu, s);
+      if (e == hipSuccess) e = gemm_launch(W.gemm(1, rows, h0, b1, nullptr, act, abuf, dtype), ncu, s);
       if (e == hipSuccess)
-        e = lne.launch(g(rows, H, FF, abuf, w2, b2, h0, GP_ACT_NONE, oc), ga2, be2, eps, ncu, s);
+        e = lne.launch(W.gemm(2, rows, abuf, b2, h0, GP_ACT_NONE, oc, dtype), ga2, be2, eps, ncu, s);
       if (e != hipSuccess) return fail_hip(e, "bert_addln_ffn launch");
       continue;
     }
-    e = gemm_launch(g(rows, H, H, at_row(attn, r0, H), w0, b0, at_row(x, r0, H), GP_ACT_NONE, ybuf), ncu, s);
+    e = gemm_launch(W.gemm(0, rows, at_row(attn, r0, H), b0, at_row(x, r0, H), GP_ACT_NONE, ybuf, dtype), ncu, s);
     if (e == hipSuccess) e = layer_norm_launch(rows, H, ybuf, ga0, be0, eps, h0, ncu, s);
-    if (e == hipSuccess) e = gemm_launch(g(rows, FF, H, h0, w1, b1, nullptr, act, abuf), ncu, s);
-    if (e == hipSuccess) e = gemm_launch(g(rows, H, FF, abuf, w2, b2, h0, GP_ACT_NONE, ybuf), ncu, s);
+    if (e == hipSuccess) e = gemm_launch(W.gemm(1, rows, h0, b1, nullptr, act, abuf, dtype), ncu, s);
+    if (e == hipSuccess) e = gemm_launch(W.gemm(2, rows, abuf, b2, h0, GP_ACT_NONE, ybuf, dtype), ncu, s);
     if (e == hipSuccess) e = layer_norm_launch(rows, H, ybuf, ga2, be2, eps, (char*)out + r0 * H * 2, ncu, s);
     if (e != hipSuccess) return fail_hip(e, "bert_addln_ffn launch");
   }

@@ -13,8 +13,9 @@
 // Kernel design.
 //  * B is consumed in its own [K][N] layout, its fragments read with the
 //    transposing LDS read (the BROW kernels) -- or, where its width or alignment
-//    does not allow that, transposed and padded (Bt[N][K], from prep_kernel), so
-//    that both MFMA operands are rows of consecutive k.  The product is computed transposed,
+//    does not allow that or the copy is the faster way (gemm_copy_weights),
+//    transposed and padded (Bt[N][K], from prep_kernel), so that both MFMA
+//    operands are rows of consecutive k.  The product is computed transposed,
 //    C^T = Bt A^T, with v_mfma_f32_32x32x16_f16: the MFMA A operand is a
 //    32-feature block of Bt, the MFMA B operand a 32-row block of A, and each
 //    accumulator lane ends up holding 4 consecutive features of one row.
@@ -761,8 +762,10 @@ template <typename E>
 static hipError_t launch_typed(const GemmArgs& a, Args& g, bool brow, int num_cus, hipStream_t s) {
   if (a.ln) {
     if (a.N == 128 && (a.M + Narrow::BM - 1) / Narrow::BM < num_cus)
-      return launch<Short, ACT_NONE, true, true, 1, E>(g, num_cus, s);
-    if (a.N == 128) return launch<Narrow, ACT_NONE, true, true, 1, E>(g, num_cus, s);
+      return brow ? launch<Short, ACT_NONE, true, true, 1, E>(g, num_cus, s)
+                  : launch<Short, ACT_NONE, true, false, 1, E>(g, num_cus, s);
+    if (a.N == 128) return brow ? launch<Narrow, ACT_NONE, true, true, 1, E>(g, num_cus, s)
+                                : launch<Narrow, ACT_NONE, true, false, 1, E>(g, num_cus, s);
     return launch<Wide, ACT_NONE, true, true, 2, E>(g, num_cus, s);
   }
   if (a.N % Wide::BN == 0) return brow ? dispatch<Wide, true, E>(g, a.act, num_cus, s) : dispatch<Wide, false, E>(g, a.act, num_cus, s);
@@ -849,9 +852,9 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t s) {
          (const half_t*)a.gamma, (const half_t*)a.beta, a.eps, nullptr, nullptr, QueueCtx{}, 0};
   if (a.dtype != GP_DTYPE_F16 && a.dtype != GP_DTYPE_BF16) return hipErrorInvalidValue;
   if (a.ln) {
-    // N = 128 (rows within a wave) or 256 .. 1024 in whole 256-feature tiles;
-    // the weights in place.
-    if (!brow || a.act != ACT_NONE || a.N > 1024 || (a.N != 128 && a.N % Wide::BN) || ((uintptr_t)a.gamma | (uintptr_t)a.beta) % 8)
+    // N = 128 (rows within a wave) or 256 .. 1024 in whole 256-feature tiles,
+    // those with the weights in place.
+    if ((!brow && a.N != 128) || a.act != ACT_NONE || a.N > 1024 || (a.N != 128 && a.N % Wide::BN) || ((uintptr_t)a.gamma | (uintptr_t)a.beta) % 8)
       return hipErrorInvalidValue;
     if (a.N != 128) {
       if (!a.ln_ws || !a.status || a.epoch == 0 || a.M > gemm_ln_max_rows(a.N, num_cus)) return hipErrorInvalidValue;
@@ -868,6 +871,12 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t s) {
   if (!a.ln)
     if (const int size = tile_cost(a.M, a.N, a.K, num_cus).size) return tile_launch(g, a.act, size, a.dtype, s);
   return a.dtype == GP_DTYPE_BF16 ? launch_typed<BF16>(a, g, brow, num_cus, s) : launch_typed<F16>(a, g, brow, num_cus, s);
+}
+
+bool gemm_copy_weights(int64_t M, int64_t rows, int64_t N, int64_t K, bool ln, int num_cus) {
+  using namespace gemm;
+  return N % Wide::BN != 0 && 2.0 * M * N * K >= 8e10 && K >= (N == 128 ? 4096 : 512) &&
+         (ln || tile_cost(rows, N, K, num_cus).size == 0);
 }
 
 bool gemm_ln_apart(int64_t M, int64_t N, int64_t K, int num_cus) {

@@ -116,7 +116,8 @@ hipError_t layer_norm_launch(int64_t M, int64_t D, const void* x, const void* ga
 hipError_t add_launch(int64_t M, int64_t N, const void* a, const void* b, void* c, int num_cus, hipStream_t stream);
 
 // Wide GEMM stage: out = act(x W + b) or x W + b + r, N a multiple of 128,
-// K a multiple of 64, with W passed transposed (wt = W^T, [N, K]).  Row
+// K a multiple of 64, with W passed transposed (wt = W^T, [N, K]) or as it is
+// (w).  Row
 // strides (elements, multiples of 8) default to K / N / N when 0; out may be a
 // column block of a wider matrix.
 struct GemmArgs {
@@ -172,19 +173,23 @@ bool gemm_ln_apart(int64_t M, int64_t N, int64_t K, int num_cus);
 // gamma / beta may be null (1 / 0).  In place when out == x.
 hipError_t gemm_ln_rows_launch(int64_t M, int64_t N, const void* x, const void* gamma, const void* beta, float eps,
                                void* out, int dtype, hipStream_t s);
-// GEMM arguments for W [K, N] read in place (row stride N).  Every 16-byte
-// aligned weight of a width that is a multiple of 128 is read this way: two
-// transposing LDS reads a fragment instead of one 16-byte read cost the K loop
-// nothing measurable (16384 x 1024 x 4096 117.9 us either way, 65536 x 1024 x
-// 1024 138.3 from a transposed copy, 140.5 in place), and the copy was a launch
-// of 7 to 14 us per call: BERT-large FFN, 65,536 rows, 1140 -> 1126 us, DLRM
-// bottom + top, 262,144 rows, 1394 -> 1364 us.
-inline GemmArgs gemm_w(int64_t M, int64_t N, int64_t K, const void* x, const void* w, const void* b, const void* r,
-                       int act, void* out) {
-  GemmArgs g{M, N, K, x, nullptr, b, r, act, out};
-  g.w = w;
-  return g;
-}
+// Whether a call of M rows, `rows` to a launch, copies a layer's weights
+// transposed into its workspace before the GEMMs that read them (wt).  In place
+// a fragment takes two transposing LDS reads instead of one 16-byte read.  The
+// 256-wide tiles read each fragment for four row blocks and hide that
+// (16384 x 1024 x 4096 117.9 us either way, 65536 x 1024 x 1024 138.3 from a
+// copy, 140.5 in place); the 128-wide tiles of an odd multiple of 128 features
+// read it for two and lose up to a seventh of a deep K walk.  The copy is a
+// launch of 3 to 14 us, which a large call of a deep layer earns back.  Copy /
+// in place, us a call (fp16, 256-row tiles):
+//   262,143 x 1024 x 384   249 / 265     262,143 x 512 x 640    247 / 254
+//   262,143 x 2048 x 384   431 / 477     180,000 x 512 x 384    114 / 116
+//    50,001 x 4096 x 1152  465 / 521     262,143 x 256 x 640    183 / 182
+//   100,003 x 8192 x 384   669 / 761      50,001 x 1024 x 1152  136 / 136
+//   100,003 x 4096 x 128   177 / 185     262,143 x 2048 x 128   217 / 213
+// Not where the call runs on the small tiles (20,011 x 8192 x 128 127 / 98),
+// which a launch that ends in a LayerNorm (ln) of 128-wide rows never does.
+bool gemm_copy_weights(int64_t M, int64_t rows, int64_t N, int64_t K, bool ln, int num_cus);
 // out[m] = act(a[m, 0:K] . w[0:K] + b[0]) for m < M (a one-output layer); K
 // and lda multiples of 8, a and w 16-byte aligned, b may be null.
 hipError_t gemv1_launch(int64_t M, int64_t K, const void* a, int64_t lda, const void* w, const void* b, int act,

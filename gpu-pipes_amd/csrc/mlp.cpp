@@ -10,8 +10,8 @@
 // here every layer is one launch of the wide GEMM stage (gemm.hip) with its
 // bias and activation fused, over row chunks of 262,144.
 // Narrow and odd widths are handled by padding, never by special kernels:
-//   * weights that the GEMM cannot read in place (in_place below) are transposed
-//     into the workspace with zero rows and columns up to K a multiple of 64 and
+//   * weights that the GEMM cannot or does not read in place (in_place below)
+//     are transposed into the workspace with zero rows and columns up to K a multiple of 64 and
 //     N a multiple of 128, their biases zero-padded to N;
 //   * an input whose width is not a multiple of 8 (or not 16-byte aligned) is
 //     copied into a padded buffer; other inputs are read in place, and the
@@ -69,9 +69,10 @@ struct Prepared {
   int64_t kw = 0;
 };
 
-// A layer reads its weights in place when its output width is a multiple of
-// 128 and weights and bias are 16-byte aligned; otherwise they are prepared
-// (transposed, zero-padded) into the workspace by the chain's prep launch.
+// A layer can read its weights in place when its output width is a multiple of
+// 128 and weights and bias are 16-byte aligned; otherwise (and where that is
+// slower, gemm_copy_weights) they are prepared -- transposed, zero-padded --
+// into the workspace by the chain's prep launch.
 bool in_place(int64_t N, const void* w, const void* b) {
   return N % 128 == 0 && aligned16(w) && (!b || aligned16(b));
 }
@@ -168,7 +169,7 @@ int run_chain(int64_t M, int nl, const int64_t* widths, const void* const* w, co
   std::vector<Prepared> L(nl);
   std::vector<PrepSpec> ps;
   for (int i = 0; i < (fused_tail ? tl : nl); ++i) {
-    if (in_place(widths[i + 1], w[i], b[i])) {
+    if (in_place(widths[i + 1], w[i], b[i]) && !gemm_copy_weights(M, CH, np[i], kin[i], false, ncu)) {
       L[i] = {nullptr, b[i], kin[i], np[i], acts[i], w[i], widths[i]};
     } else {
       ps.push_back({w[i], ws + o_wt[i], b[i], ws + o_b[i], widths[i], widths[i + 1], kin[i], np[i]});

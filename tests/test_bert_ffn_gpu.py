@@ -257,6 +257,65 @@ def test_gemm_ragged_tile_counts(cuda, M, N, K, act):
     assert_parity(f(y[-300:]), oracle.linear(f(x[-300:]), f(w), f(b), ACT_ID[act]), f"gemm M={M} N={N} K={K}")
 
 
+def capture_error(call):
+    """The library's error of a call made while its stream is being captured."""
+    torch.cuda.synchronize()
+    g, err = torch.cuda.CUDAGraph(), None
+    with torch.cuda.graph(g):
+        try:
+            call()
+        except gpipes.GpipesError as e:
+            err = e
+    return err
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,resid", [(100003, 384, 1088, False), (131072, 640, 512, True), (131071, 128, 4096, False)])
+def test_gemm_deep_narrow_layers_copy_their_weights(cuda, M, N, K, resid, dtype):
+    """Large calls of an odd multiple of 128 features and a deep K read a
+    transposed copy of the weights (in place costs their 128-wide tiles up to a
+    seventh of the K walk): such a call needs the workspace, which capture refuses,
+    and gives the bits of the same rows in calls that read the weights in place."""
+    x = normal_fp16(M, K, seed=N, device=cuda, dtype=dtype)
+    w = (normal_fp16(K, N, seed=K, device=cuda).float() / K ** 0.5).to(dtype)
+    b = normal_fp16(1, N, seed=3, device=cuda, dtype=dtype)[0]
+    r = normal_fp16(M, N, seed=4, device=cuda, dtype=dtype) if resid else None
+    act = "none" if resid else "gelu_tanh"
+    out = torch.full((M, N), float("nan"), dtype=dtype, device=cuda)
+    gpipes.gemm_out(x, w, b, r, act=act, out=out)
+    assert not torch.isnan(out).any()
+    for r0 in (0, M // 2, M - 5001):
+        part = gpipes.gemm_out(x[r0:r0 + 5001].clone(), w, b, None if r is None else r[r0:r0 + 5001].clone(), act=act)
+        assert torch.equal(out[r0:r0 + 5001].view(torch.int16), part.view(torch.int16)), r0
+    err = capture_error(lambda: gpipes.gemm_out(x, w, b, r, act=act, out=out))
+    assert err is not None and err.code == -1 and "workspace" in str(err)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H,FF", [(128, 8192), (512, 640)])
+def test_ffn_with_copied_weights_matches_small_batches(cuda, H, FF, dtype):
+    """The FFN blocks whose second (H 128, deep FF) or first layer (odd multiple
+    of 128 features) reads a transposed copy in a large call: the bits of a small
+    batch, which reads them in place."""
+    M = 130001 if H == 512 else 40001
+    p = {k: v.to(dtype) for k, v in dev(bert_params(H, FF, seed=H, init="torch", affine_random=True), cuda).items()}
+    w0 = (normal_fp16(H, H, seed=2, device=cuda).float() / H ** 0.5).to(dtype)
+    a, x = normal_fp16(M, H, seed=5, device=cuda, dtype=dtype), normal_fp16(M, H, seed=6, device=cuda, dtype=dtype)
+    f_p = (p["w1"], p["b1"], p["w2"], p["b2"])
+    ga = (p["gamma"], p["beta"])
+
+    def ffn_(n):
+        return gpipes.bert_ffn(x[n], *f_p, *ga, act="relu")
+
+    def addln(n):
+        return gpipes.bert_addln_ffn(a[n], x[n], w0, p["b2"], *f_p, *ga, *ga, act="relu")
+
+    for call in (ffn_, addln):
+        big = call(slice(0, M))
+        for n in (slice(0, 65), slice(M // 2, M // 2 + 700), slice(M - 300, M)):
+            assert torch.equal(call(n).view(torch.int16), big[n].view(torch.int16)), n
+
+
 def test_gemm_identity_weight_is_exact(cuda):
     """x . I (+ 0) passes every fp16 value through the fp32 accumulator unchanged."""
     M, K = 700, 256

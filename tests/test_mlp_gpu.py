@@ -331,3 +331,18 @@ def test_nerf_few_rows_match_many(cuda, Kx, Kd, Na, Nrgb, dtype):
         got = gpipes.nerf_full(x[:m], d[:m], *wb, rgb_act="sigmoid") + (gpipes.nerf_a(x[:m], *wb[:16]),)
         for y, b, t in zip(got, big, tail):
             assert torch.equal(bits(y[:65536]), bits(b)) and torch.equal(bits(y[65536:]), bits(t[:n])), m
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_mlp_copied_weights_match_small_calls(cuda, dtype):
+    """Layers of an odd multiple of 128 features and a deep K read a transposed
+    copy of their weights in a large call, and the weights in place in a small one:
+    the same bits.  (599 is padded to K 640.)"""
+    M, widths, acts = 140000, [599, 896, 640, 5], ["relu", "gelu_tanh", "none"]
+    ws, bs = dlrm_params(widths, seed=7, init="xavier")
+    ws, bs = [w.to(dtype).to(cuda) for w in ws], [b.to(dtype).to(cuda) for b in bs]
+    x = normal_fp16(M, widths[0], seed=8, device=cuda, dtype=dtype)
+    big = gpipes.mlp_out(x, ws, bs, acts)
+    for r0 in (0, 70001, M - 3000):
+        small = gpipes.mlp_out(x[r0:r0 + 3000].clone(), ws, bs, acts)
+        assert torch.equal(small.view(torch.int16), big[r0:r0 + 3000].view(torch.int16)), r0
