@@ -105,6 +105,8 @@ int run_mgn(const MgnArgs& a, int impl, hipStream_t stream) {
   if (a.dtype != GP_DTYPE_F16 && a.dtype != GP_DTYPE_BF16) return fail(GP_ERR_INVALID_ARG, "unknown dtype %d", a.dtype);
   if (a.dtype == GP_DTYPE_BF16 && impl != GP_IMPL_FUSED)
     return fail(GP_ERR_INVALID_ARG, "bf16 runs on the fused kernel (impl %d) only", GP_IMPL_FUSED);
+  if (a.fresh_out && impl != GP_IMPL_FUSED)
+    return fail(GP_ERR_INVALID_ARG, "GP_OUT_FRESH applies to the fused kernel (impl %d) only", GP_IMPL_FUSED);
   if (a.M == 0) return GP_OK;
   int dev = 0, ncu = 0;
   rc = current_device_info(&dev, &ncu);
@@ -158,7 +160,8 @@ int gp_mgn_mlp_dtype_out(int64_t M, int64_t K, const void* x, const void* w1, co
                          const void* b2, const void* w3, const void* b3, const void* gamma, const void* beta,
                          float eps, void* out, int impl, int dtype, void* stream) {
   MgnArgs a{M, K, x, w1, b1, w2, b2, w3, b3, gamma, beta, eps, out};
-  a.dtype = dtype;
+  a.dtype = dtype & ~GP_OUT_FRESH;
+  a.fresh_out = (dtype & GP_OUT_FRESH) != 0;
   return run_mgn(a, impl, (hipStream_t)stream);
 }
 

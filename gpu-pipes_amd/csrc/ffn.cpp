@@ -73,6 +73,7 @@ struct LnEpilogue {
   void* ws = nullptr;
   uint32_t epoch = 0;
   int64_t round = 0;
+  bool fresh_out = false;  // GP_OUT_FRESH
 
   // exchange: some launch of the call runs its LayerNorm in the epilogue.
   // Without one the call only registers itself (a clean status word), so that
@@ -91,6 +92,7 @@ struct LnEpilogue {
   }
   GemmArgs apply(GemmArgs g, const void* gamma, const void* beta, float eps) {
     g.ln = 1;
+    g.fresh_out = fresh_out;
     g.gamma = gamma;
     g.beta = beta;
     g.eps = eps;
@@ -211,6 +213,8 @@ int gp_bert_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* x, const
                           void* out, int dtype, void* stream) {
   clear_error();
   int rc;
+  const bool fresh_out = dtype & GP_OUT_FRESH;
+  dtype &= ~GP_OUT_FRESH;
   if ((rc = check_dtype(dtype))) return rc;
   if (M < 0) return fail(GP_ERR_INVALID_ARG, "M must be >= 0 (got %lld)", (long long)M);
   if (H != 128 && H != 256 && H != 512 && H != 1024)
@@ -257,6 +261,7 @@ int gp_bert_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* x, const
   hipError_t e = W.copy(s);
   if (e != hipSuccess) return fail_hip(e, "transpose launch");
   LnEpilogue lne;
+  lne.fresh_out = fresh_out;
   if (fuse_ln && (rc = lne.init(dev, s, CH, H, !gemm_ln_apart(CH, H, FF, ncu)))) return rc;
   for (int64_t r0 = 0; r0 < M; r0 += CH) {
     const int64_t rows = M - r0 < CH ? M - r0 : CH;
@@ -317,7 +322,11 @@ int gp_bert_addln_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* at
                                 float eps, int act, void* out, int impl, int dtype, void* stream) {
   clear_error();
   int rc;
+  const bool fresh_out = dtype & GP_OUT_FRESH;
+  dtype &= ~GP_OUT_FRESH;
   if ((rc = check_dtype(dtype))) return rc;
+  if (fresh_out && impl != GP_IMPL_FUSED)
+    return fail(GP_ERR_INVALID_ARG, "GP_OUT_FRESH applies to the fused implementation (impl %d) only", GP_IMPL_FUSED);
   if (dtype != GP_DTYPE_F16 && impl != GP_IMPL_FUSED)
     return fail(GP_ERR_INVALID_ARG, "bf16 runs the fused implementation only (the queue-chained layout is fp16)");
   if (M < 0) return fail(GP_ERR_INVALID_ARG, "M must be >= 0 (got %lld)", (long long)M);
@@ -374,6 +383,7 @@ int gp_bert_addln_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* at
   hipError_t e = W.copy(s);
   if (e != hipSuccess) return fail_hip(e, "transpose launch");
   LnEpilogue lne;
+  lne.fresh_out = fresh_out;
   if (fuse_ln && (rc = lne.init(dev, s, CH, H, !gemm_ln_apart(CH, H, H, ncu) || !gemm_ln_apart(CH, H, FF, ncu)))) return rc;
   for (int64_t r0 = 0; r0 < M; r0 += CH) {
     const int64_t rows = M - r0 < CH ? M - r0 : CH;

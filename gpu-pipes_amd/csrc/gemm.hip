@@ -554,7 +554,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         }
       }
       // Pass 3: normalise, affine, fp16, store.  After a failed wait nothing
-      // is stored.
+      // is stored, or zeros where the output holds nothing yet.
       if (ok) {
 #pragma unroll
         for (int nb = 0; nb < C::NBW; ++nb) {
@@ -575,6 +575,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 1))) void
             store_frag(o, nb, mb);
           }
         }
+      } else if (p.fresh_out) {
+        const u32x2 zero[4] = {};
+        for (int nb = 0; nb < C::NBW; ++nb)
+#pragma unroll
+          for (int mb = 0; mb < C::MBW; ++mb) store_frag(zero, nb, mb);
       }
 #pragma unroll
       for (int nb = 0; nb < C::NBW; ++nb)
@@ -849,7 +854,7 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t s) {
   if (!brow && !a.wt) return hipErrorInvalidValue;
   Args g{(const half_t*)a.x, (const half_t*)a.wt, (const half_t*)a.w, ldw, kw, (const half_t*)a.b,
          (const half_t*)a.r, (half_t*)a.out, a.M, (int)a.N, (int)a.K, ka, lda, ldc, ldr,
-         (const half_t*)a.gamma, (const half_t*)a.beta, a.eps, nullptr, nullptr, QueueCtx{}, 0};
+         (const half_t*)a.gamma, (const half_t*)a.beta, a.eps, nullptr, nullptr, QueueCtx{}, 0, a.fresh_out};
   if (a.dtype != GP_DTYPE_F16 && a.dtype != GP_DTYPE_BF16) return hipErrorInvalidValue;
   if (a.ln) {
     // N = 128 (rows within a wave) or 256 .. 1024 in whole 256-feature tiles,

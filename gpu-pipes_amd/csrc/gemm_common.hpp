@@ -43,6 +43,7 @@ struct Args {
   QCounter* cnt;
   QueueCtx ctx;
   uint32_t ln_target;  // count of a row block's counter once this launch's waves have all committed
+  int fresh_out;       // LNM 2: zeros for the rows of a failed wait
 };
 
 // Small-tile kernels (gemm_tile.hip): one `size` x `size` output tile per

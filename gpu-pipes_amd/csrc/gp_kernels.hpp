@@ -40,6 +40,9 @@ struct MgnArgs {
   uint32_t epoch = 0;
   int spin_limit = 0;
   int dtype = GP_DTYPE_F16;  // element type of x, the weights and out (GP_DTYPE_BF16: fused kernel only)
+  // The fused kernel, after a failed wait: rows it does not compute are zeroed
+  // (GP_OUT_FRESH) instead of left as they were.
+  bool fresh_out = false;
 };
 
 // Persistent fused kernel (all layers in one workgroup per CU).
@@ -147,7 +150,10 @@ struct GemmArgs {
   // num_cus is a multiple of N / 256, else one) and at most 1024 row blocks.  Launches of one epoch on
   // one ln_ws are numbered by ln_round (0, 1, ...) and must cover a prefix of
   // the same row blocks in every earlier round.
+  // After a failed wait the rows that are not computed are left as they were, or
+  // with fresh_out zeroed.
   int ln = 0;
+  bool fresh_out = false;
   int64_t ln_round = 0;
   int dtype = GP_DTYPE_F16;  // element type of x, the weights, b, r, gamma, beta and out
   const void* gamma = nullptr;

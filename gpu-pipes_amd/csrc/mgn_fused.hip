@@ -91,6 +91,7 @@ struct Params {
   unsigned long long* status;
   uint32_t epoch;
   int spin_limit;
+  int fresh_out;  // an aborted workgroup's rows read as zeros, not as they were
 };
 
 // LDS synchronisation words (monotonic counters, one count per wave per tile).
@@ -705,6 +706,17 @@ void mgn_fused_kernel(Params p) {
       tile_b((GP_LDS char*)hand0, k);
       if (k + 1 < nt) tile_b((GP_LDS char*)hand1, k + 1);
     }
+    // A wave that skipped a store saw the abort word, which stays set: it zeroes
+    // its sixteen rows of every tile, behind the stores it did issue.
+    if (p.fresh_out && lds_load_relaxed(ab) != 0) {
+      wait_vmcnt<0>();
+      for (int k = 0; k < nt; ++k) {
+        const int64_t grow = (t0 + (int64_t)k * G) * TM + 16 * n + l16;
+        const h4 zero[2] = {};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) store_row_pair(p.out + grow * D, zero, j, q4, grow < M);
+      }
+    }
     pt.finish(wave, lane, nt, t_entry, pro_t);
   }
   // The abort word is sticky and is set before the wave that set it gets
@@ -722,7 +734,7 @@ static hipError_t launch_fused(const MgnArgs& a, int grid, hipStream_t stream) {
   fused::Params p{(const half_t*)a.x,  (const half_t*)a.w1, (const half_t*)a.b1, (const half_t*)a.w2,
                   (const half_t*)a.b2, (const half_t*)a.w3, (const half_t*)a.b3, (const half_t*)a.gamma,
                   (const half_t*)a.beta, (half_t*)a.out, a.M, a.eps, (const half_t*)a.nf, a.N, a.src, a.dst,
-                  a.status, a.epoch, a.spin_limit > 0 ? a.spin_limit : kSpinLimit};
+                  a.status, a.epoch, a.spin_limit > 0 ? a.spin_limit : kSpinLimit, a.fresh_out};
   hipLaunchKernelGGL((fused::mgn_fused_kernel<K, LN, GI, E>), dim3(grid), dim3(fused::NTHREADS), 0, stream, p);
   return hipGetLastError();
 }

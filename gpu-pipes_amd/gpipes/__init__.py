@@ -127,9 +127,12 @@ def _check(rc):
         raise GpipesError(rc, lib.gp_last_error().decode())
 
 
-# The allocating forms leave their outputs uninitialised (the reference zeroes
+# The allocating forms do not fill their outputs first (the reference zeroes
 # them): the kernels write every row, and the fill was a pass over the output --
-# 14 us of the 57 us that a 262,144-row MGN node MLP took.
+# 14 us of the 57 us that a 262,144-row MGN node MLP took.  Rows that a launch
+# leaves out because a device-side wait failed read as zeros all the same: the
+# fused kernels that wait write them themselves (_FRESH, GP_OUT_FRESH), and the
+# queue-chained layouts get a filled output (_new).  The others wait for nothing.
 #
 # The host side of a call: about thirty attribute checks, a device guard and a
 # stream lookup.  torch.cuda.device() and torch.cuda.current_stream() cost
@@ -210,6 +213,15 @@ def _same_device(*ts):
 
 
 _DTYPES = {torch.float16: 0, torch.bfloat16: 1}  # GP_DTYPE_F16, GP_DTYPE_BF16
+_FRESH = 0x100  # GP_OUT_FRESH
+
+
+def _new(x, impl, cols=None):
+    """Output of an allocating form with x's rows: `cols` wide, or as wide as x."""
+    fused = _IMPLS.get(impl, impl) == IMPL_FUSED
+    if cols is None:
+        return torch.empty_like(x) if fused else torch.zeros_like(x)
+    return (torch.empty if fused else torch.zeros)((x.shape[0], cols), dtype=x.dtype, device=x.device)
 
 
 def mgn_mlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps=1e-5, impl="fused"):
@@ -219,6 +231,10 @@ def mgn_mlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps=1e-5, impl="fus
     Every tensor is float16, or every tensor is bfloat16 (fused impl only:
     gp_mgn_mlp_dtype_out).
     """
+    return _mgn_mlp(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps, impl, 0)
+
+
+def _mgn_mlp(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps, impl, fresh):
     if not isinstance(x, torch.Tensor) or x.dim() != 2:
         raise RuntimeError("x must be a 2-D tensor [M, K]")
     M, K = x.shape
@@ -241,45 +257,48 @@ def mgn_mlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps=1e-5, impl="fus
     with _on(x):
         args = (M, K, _ptr(x), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(w3), _ptr(b3), _ptr(gamma),
                 _ptr(beta), float(eps), _ptr(out), int(impl_id))
-        if dt == torch.float16:
-            rc = lib.gp_mgn_mlp_out(*args, _stream(x))
-        else:
-            rc = lib.gp_mgn_mlp_dtype_out(*args, _DTYPES[dt], _stream(x))
+        if impl_id != IMPL_FUSED:
+            fresh = 0
+        rc = lib.gp_mgn_mlp_dtype_out(*args, _DTYPES[dt] | fresh, _stream(x))
     _check(rc)
     return out
 
 
 def mgn_mlp(x, w1, b1, w2, b2, w3, b3, gamma=None, beta=None, eps=1e-5, impl="fused"):
-    out = torch.empty((x.shape[0], 128), dtype=x.dtype, device=x.device)
-    return mgn_mlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps=eps, impl=impl)
+    out = _new(x, impl, 128)
+    return _mgn_mlp(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps, impl, _FRESH)
+
+
+def _check_edge_input(x):
+    _check_input("x", x)
+    if x.dim() != 2 or x.shape[1] != 384:
+        raise RuntimeError("x must be [M, 384]")
 
 
 def mgn_fullmlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out):
     """Edge MLP 384->128->128->128 + LayerNorm(eps=1e-5) into ``out``
     (mgn_fullmlp_pl_ext.cu:24-71)."""
-    _check_input("x", x)
-    if x.dim() != 2 or x.shape[1] != 384:
-        raise RuntimeError("x must be [M, 384]")
+    _check_edge_input(x)
     return mgn_mlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps=1e-5)
 
 
 def mgn_fullmlp(x, w1, b1, w2, b2, w3, b3, gamma, beta):
     """Allocating form: returns a new [M, 128] tensor (mgn_fullmlp_pl_ext.cu:74-88)."""
-    out = torch.empty((x.shape[0], 128), dtype=x.dtype, device=x.device)
-    return mgn_fullmlp_out(x, w1, b1, w2, b2, w3, b3, gamma, beta, out)
+    out = _new(x, "fused", 128)
+    _check_edge_input(x)
+    return _mgn_mlp(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, 1e-5, "fused", _FRESH)
 
 
 def mgn_linears_out(x, w1, b1, w2, b2, w3, b3, out):
     """384->128->128->128 without LayerNorm (mgn_linears_pl_ext.cu:24-66)."""
-    _check_input("x", x)
-    if x.dim() != 2 or x.shape[1] != 384:
-        raise RuntimeError("x must be [M, 384]")
+    _check_edge_input(x)
     return mgn_mlp_out(x, w1, b1, w2, b2, w3, b3, None, None, out)
 
 
 def mgn_linears(x, w1, b1, w2, b2, w3, b3):
-    out = torch.empty((x.shape[0], 128), dtype=x.dtype, device=x.device)
-    return mgn_linears_out(x, w1, b1, w2, b2, w3, b3, out)
+    out = _new(x, "fused", 128)
+    _check_edge_input(x)
+    return _mgn_mlp(x, w1, b1, w2, b2, w3, b3, None, None, out, 1e-5, "fused", _FRESH)
 
 
 # ---------------------------------------------------------------------------
@@ -611,6 +630,10 @@ def bert_ffn_out(x, w1, b1, w2, b2, ga, be, out, eps=1e-5, act="relu", impl="fus
     tensor float16, or every tensor bfloat16 (gp_bert_ffn_dtype_out).  impl="pipelined"
     runs the reference app's queue-chained layout (gp_bert_ffn_impl_out; H 128, FF 512,
     ReLU or GELU(tanh), float16)."""
+    return _bert_ffn(x, w1, b1, w2, b2, ga, be, out, eps, act, impl, 0)
+
+
+def _bert_ffn(x, w1, b1, w2, b2, ga, be, out, eps, act, impl, fresh):
     dt = _dtype_of(x)
     _check_input("x", x, dtype=dt)
     if x.dim() != 2:
@@ -631,8 +654,8 @@ def bert_ffn_out(x, w1, b1, w2, b2, ga, be, out, eps=1e-5, act="relu", impl="fus
     with _on(x):
         if impl_id == IMPL_FUSED:
             _check(lib.gp_bert_ffn_dtype_out(M, H, FF, _ptr(x), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(ga),
-                                             _ptr(be), float(eps), ACTS.get(act, act), _ptr(out), _DTYPES[dt],
-                                             _stream(x)))
+                                             _ptr(be), float(eps), ACTS.get(act, act), _ptr(out),
+                                             _DTYPES[dt] | fresh, _stream(x)))
         else:
             if dt != torch.float16:
                 raise RuntimeError("the pipelined layout takes float16 tensors only")
@@ -644,8 +667,8 @@ def bert_ffn_out(x, w1, b1, w2, b2, ga, be, out, eps=1e-5, act="relu", impl="fus
 
 def bert_ffn(x, w1, b1, w2, b2, ga, be, eps=1e-5, act="relu", impl="fused"):
     """Allocating form (bert_ffn_pl_ext.cu:59-72)."""
-    out = torch.empty_like(x)
-    return bert_ffn_out(x, w1, b1, w2, b2, ga, be, out, eps=eps, act=act, impl=impl)
+    out = _new(x, impl)
+    return _bert_ffn(x, w1, b1, w2, b2, ga, be, out, eps, act, impl, _FRESH)
 
 
 # ---------------------------------------------------------------------------
@@ -749,6 +772,10 @@ def bert_addln_ffn_out(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, 
     GEMM launch per layer with fused epilogues) or "pipelined" (the reference's queue-chained
     layout, H 128 / FF 512 only).  Every tensor float16, or every tensor bfloat16 (fused impl
     only: gp_bert_addln_ffn_dtype_out)."""
+    return _bert_addln_ffn(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, out, eps, act, impl, 0)
+
+
+def _bert_addln_ffn(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, out, eps, act, impl, fresh):
     dt = _dtype_of(attn_out)
     _check_input("attn_out", attn_out, dtype=dt)
     if attn_out.dim() != 2:
@@ -771,16 +798,15 @@ def bert_addln_ffn_out(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, 
         _check(lib.gp_bert_addln_ffn_dtype_out(M, H, FF, _ptr(attn_out), _ptr(x), _ptr(w0), _ptr(b0), _ptr(w1),
                                                _ptr(b1), _ptr(w2), _ptr(b2), _ptr(ga0), _ptr(be0), _ptr(ga2),
                                                _ptr(be2), float(eps), ACTS.get(act, act), _ptr(out), int(impl_id),
-                                               _DTYPES[dt], _stream(x)))
+                                               _DTYPES[dt] | (fresh if impl_id == IMPL_FUSED else 0), _stream(x)))
     return out
 
 
 def bert_addln_ffn(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, eps=1e-5, act="relu", impl="fused"):
     """Allocating form (bert_addln_ffn_pl_ext.cu:61-76, which passes be0 for be2 -- not
     reproduced: ga2 / be2 are used as given)."""
-    out = torch.empty_like(x)
-    return bert_addln_ffn_out(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, out, eps=eps, act=act,
-                              impl=impl)
+    out = _new(x, impl)
+    return _bert_addln_ffn(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, out, eps, act, impl, _FRESH)
 
 
 def nerf_a_out(x, *wb_and_out, impl="fused"):
@@ -815,8 +841,7 @@ def nerf_a(x, *wb, impl="fused"):
     """Allocating form: returns a new [M, 256] tensor (nerf_a_pl_ext.cu:79-110)."""
     if len(wb) != 16:
         raise RuntimeError("expected w1, b1, ..., w8, b8")
-    out = torch.empty((x.shape[0], 256), dtype=x.dtype, device=x.device)
-    return nerf_a_out(x, *wb, out, impl=impl)
+    return nerf_a_out(x, *wb, _new(x, impl, 256), impl=impl)
 
 
 def nerf_full_out_noalloc(x, d, *wb_and_outs, rgb_act="none"):

@@ -44,6 +44,13 @@ extern "C" {
 /* Element types of the *_dtype_out entry points (16-bit storage, fp32 accumulation). */
 #define GP_DTYPE_F16 0  /* IEEE binary16 */
 #define GP_DTYPE_BF16 1 /* bfloat16      */
+/* Or-ed into the dtype of gp_mgn_mlp_dtype_out (GP_IMPL_FUSED),               */
+/* gp_bert_ffn_dtype_out and gp_bert_addln_ffn_dtype_out (GP_IMPL_FUSED): out  */
+/* is memory that nothing has been written to.  What a launch that fails on    */
+/* the device (GP_ERR_TIMEOUT) does not compute of it then reads as zeros, at  */
+/* no cost to a launch that succeeds; without the flag a failed launch leaves  */
+/* that part of out as it was.                                                 */
+#define GP_OUT_FRESH 0x100
 
 /* Activations of gp_linear_out. */
 #define GP_ACT_NONE 0

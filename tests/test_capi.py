@@ -96,6 +96,12 @@ def test_wide_dtype_entry_points_reject_before_any_device_call():
     args12 = [vp(16)] * 12
     assert L.gp_bert_addln_ffn_dtype_out(16, 128, 512, *args12, 1e-5, 1, vp(16), 1, 1, None) == -1  # bf16 + pipelined
     assert L.gp_bert_addln_ffn_dtype_out(16, 128, 512, *args12, 1e-5, 1, vp(16), 0, 3, None) == -1
+    fresh = 0x100  # GP_OUT_FRESH: with the fused implementations only, and not a dtype of its own
+    assert L.gp_bert_addln_ffn_dtype_out(16, 128, 512, *args12, 1e-5, 1, vp(16), 1, fresh, None) == -1
+    assert L.gp_bert_addln_ffn_dtype_out(0, 128, 512, *args12, 1e-5, 1, vp(16), 0, fresh | 1, None) == 0
+    assert L.gp_bert_ffn_dtype_out(16, 1024, 4096, *args, 1e-12, 2, vp(16), fresh | 2, None) == -1
+    assert L.gp_bert_ffn_dtype_out(0, 1024, 4096, *args, 1e-12, 2, vp(16), fresh, None) == 0
+    assert L.gp_gemm_dtype_out(16, 256, 64, vp(16), vp(16), None, None, 0, vp(16), fresh, None) == -1
     w = (vp * 12)(*([16] * 12))
     b = (vp * 12)()
     assert L.gp_nerf_full_dtype_out(16, 64, 27, 1, 3, vp(16), vp(16), w, b, 3, vp(16), vp(16), 7, None) == -1

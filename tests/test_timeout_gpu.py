@@ -162,6 +162,99 @@ def test_route_timeout_reported(cuda, restore_limit, route):
         assert torch.equal(out2.view(torch.int16), x.view(torch.int16))
 
 
+def fresh_rows(call, ref):
+    """`call` (an allocating form) under a one-poll wait bound, its output taken
+    from memory that held sentinels: the share of the elements that are zero, all
+    others being `ref`'s."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    old = torch.full(ref.shape, SENTINEL, dtype=torch.int16, device=ref.device).view(ref.dtype)
+    at = old.data_ptr()
+    torch.cuda.synchronize()
+    del old
+    gpipes.set_wait_limit(1)
+    out = call()
+    expect_timeout()
+    gpipes.set_wait_limit(0)
+    assert out.data_ptr() == at, "the output is not the memory that held the sentinels"
+    g, r = out.view(torch.int16), ref.view(torch.int16)
+    assert bool(((g == 0) | (g == r)).all()), "neither zero nor a normal launch's value"
+    return float((g == 0).float().mean())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,ln", [(384, True), (256, False), (128, True)])
+def test_failed_mgn_launch_leaves_zeros_in_a_new_output(cuda, restore_limit, K, ln, dtype):
+    """An allocating form does not fill its output: the rows of a workgroup whose
+    wait failed read as zeros all the same, as where the output was filled first."""
+    M = 64 * 256 * 3 + 5
+    p = to_dev(mgn_params(K, seed=K, layernorm=ln, affine_random=True, dtype=dtype), cuda)
+    x = normal_fp16(M, K, seed=1, device=cuda, dtype=dtype)
+    args = (x, p["w1"], p["b1"], p["w2"], p["b2"], p["w3"], p["b3"], p["gamma"], p["beta"])
+    ref = gpipes.mgn_mlp(*args)
+    zeros = fresh_rows(lambda: gpipes.mgn_mlp(*args), ref)
+    print(f"[fresh] K={K} {dtype}: {zeros:.3f} zero", flush=True)
+    assert zeros > 0.01, "no wait failed"
+    if K == 384 and dtype == torch.float16:
+        fresh_rows(lambda: gpipes.mgn_fullmlp(*args), ref)
+    again = gpipes.mgn_mlp(*args)
+    gpipes.pipeline_check()
+    assert torch.equal(again.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block", ["bert_ffn", "bert_addln_ffn"])
+def test_failed_ln_exchange_leaves_zeros_in_a_new_output(cuda, restore_limit, block, dtype):
+    """The FFN blocks whose LayerNorm exchanges statistics between workgroups."""
+    from gpipes.synth import bert_params
+    M, H, FF = 16384, 1024, 1024
+    p = {k: v.to(cuda).to(dtype) for k, v in bert_params(H, FF, seed=2, init="bert").items()}
+    x = normal_fp16(M, H, seed=3, device=cuda, dtype=dtype)
+    ffn = (p["w1"], p["b1"], p["w2"], p["b2"])
+    ln = (p["gamma"], p["beta"])
+
+    def call():
+        if block == "bert_ffn":
+            return gpipes.bert_ffn(x, *ffn, *ln, act="relu")
+        return gpipes.bert_addln_ffn(x, x, p["w1"], p["b1"], *ffn, *ln, *ln, act="relu")
+
+    ref = call()
+    gpipes.pipeline_check()
+    if block == "bert_ffn":
+        zeros = fresh_rows(call, ref)
+        print(f"[fresh] {block} {dtype}: {zeros:.3f} zero", flush=True)
+    else:
+        # (After a failed first LayerNorm the later layers run on the rows there
+        # are: only that nothing of the old memory shows.)
+        old = torch.full_like(ref, float("nan"))
+        torch.cuda.synchronize()
+        del old
+        gpipes.set_wait_limit(1)
+        out = call()
+        expect_timeout()
+        gpipes.set_wait_limit(0)
+        assert not torch.isnan(out).any()
+    again = call()
+    gpipes.pipeline_check()
+    assert torch.equal(again.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("impl", ["pipelined", "pipelined_split_ln"])
+def test_failed_pipeline_leaves_nothing_of_the_old_memory(cuda, restore_limit, impl):
+    M, K = 128 * 300 + 7, 384
+    p = to_dev(mgn_params(K, seed=11, affine_random=True), cuda)
+    x = normal_fp16(M, K, seed=12).to(cuda)
+    torch.cuda.synchronize()
+    old = torch.full((M, 128), SENTINEL, dtype=torch.int16, device=cuda)
+    torch.cuda.synchronize()
+    del old
+    gpipes.set_wait_limit(1)
+    out = run_gpu(x, p, impl=impl)
+    expect_timeout()
+    gpipes.set_wait_limit(0)
+    assert not bool((out.view(torch.int16) == SENTINEL).any())
+
+
 def test_check_without_launch(cuda):
     """A stream that has had no reporting launch is an argument error, not a pass."""
     s = torch.cuda.Stream(device=cuda)
