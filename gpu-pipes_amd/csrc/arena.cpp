@@ -11,9 +11,10 @@
 // kernel, whose payload may lie where this one's counters are) zeroes the
 // arena once first.
 //
-// Workspaces hold the intermediates of the unpipelined wide operators (the
-// BERT FFN's transposed weights and activation chunks): one per (device,
-// stream), grown on demand, never zeroed.
+// Workspaces hold the intermediates of the unpipelined wide operators
+// (activation chunks, packed weights of the fused chains, transposed copies of
+// weights that are not read in place): one per (device, stream), grown on
+// demand, never zeroed.
 #include <hip/hip_runtime.h>
 
 #include <map>
@@ -25,13 +26,10 @@
 
 namespace gp {
 
-namespace {
-// True when work enqueued on `stream` is being captured into a graph.
 bool capturing(hipStream_t stream) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
-}  // namespace
 
 int refuse_capture(hipStream_t stream) {
   if (capturing(stream))

@@ -194,9 +194,13 @@ int gp_gemm_dtype_out(int64_t M, int64_t N, int64_t K, const void* x, const void
   Weights W(M, M, ncu);
   W.add(N, K, w, false);
   if (W.bytes && (rc = workspace_acquire(dev, s, W.bytes, (void**)&W.base))) return rc;
-  // (Calls of this much work have never been capturable: they used the
-  // workspace when the weights were still copied.)
-  if (2.0 * M * N * K >= 8e10 && (rc = refuse_capture(s))) return rc;
+  // Which of the large calls take the workspace depends on their shape and on the
+  // kernels (gemm_copy_weights); capture is refused to all of them, so that what a
+  // program may capture follows from M, N and K.
+  if (2.0 * M * N * K >= 8e10 && capturing(s))
+    return fail(GP_ERR_INVALID_ARG,
+                "GEMM calls of 8e10 FLOP (2 M N K) or more cannot be captured into a graph (by their shape, they may "
+                "need the per-stream workspace)");
   hipError_t e = W.copy(s);
   if (e != hipSuccess) return fail_hip(e, "transpose launch");
   e = gemm_launch(W.gemm(0, M, x, b, r, act, out, dtype), ncu, s);

@@ -45,6 +45,8 @@ constexpr uint32_t kArenaLayoutGemmLn = 6;  // LayerNorm-epilogue GEMMs: partial
 constexpr uint32_t kArenaLayoutBertFfn = 7;
 constexpr uint32_t kArenaLayoutMgnSplit = 8;  // mgn_pipelined's split-LayerNorm layout
 constexpr uint32_t kArenaLayoutRouteReload = 9;  // the one-slot route of 64-row entries
+// True when work enqueued on `stream` is being captured into a graph.
+bool capturing(hipStream_t stream);
 // GP_ERR_INVALID_ARG if `stream` is capturing into a graph: the queue-chained
 // launches call it before any other HIP call (a replay would reuse the
 // captured queue epoch).

@@ -376,7 +376,11 @@ int gp_linear_layer_norm_out(int64_t M, int64_t K, const void* x, const void* w,
  * residual as accumulator (apps/bert_ffn/pipelined/bert_ffn_pl.cuh:79-99,
  * common/pipe_gemm.cuh:128-146), and bulksync_gemm<M,N,K,RELU>
  * (common/bulksync_gemm.cuh:13-110) beyond the 128-wide stage of
- * gp_linear_out.  w is transposed into the per-stream workspace on each call.
+ * gp_linear_out.  w is read as it is; calls of 2 M N K >= 8e10 copy it
+ * transposed into the per-stream workspace where that is faster (N an odd
+ * multiple of 128 and a deep K).  Smaller calls allocate nothing and may be
+ * captured into a graph; calls of 8e10 or more are refused under capture
+ * (GP_ERR_INVALID_ARG).
  */
 int gp_gemm_out(int64_t M, int64_t N, int64_t K, const void* x, const void* w, const void* b, const void* r,
                 int act, void* out, void* stream);

@@ -288,7 +288,7 @@ def test_gemm_deep_narrow_layers_copy_their_weights(cuda, M, N, K, resid, dtype)
         part = gpipes.gemm_out(x[r0:r0 + 5001].clone(), w, b, None if r is None else r[r0:r0 + 5001].clone(), act=act)
         assert torch.equal(out[r0:r0 + 5001].view(torch.int16), part.view(torch.int16)), r0
     err = capture_error(lambda: gpipes.gemm_out(x, w, b, r, act=act, out=out))
-    assert err is not None and err.code == -1 and "workspace" in str(err)
+    assert err is not None and err.code == -1 and "that use the per-stream workspace" in str(err)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

@@ -8,7 +8,8 @@ the eager call on the inputs the buffers hold at replay time, bit for bit;
 the replays are interleaved with eager work, synchronisations and new input
 values.  The queue-chained implementations (a new queue epoch per launch) and
 the calls that use the per-stream workspace refuse capture with
-GP_ERR_INVALID_ARG before enqueueing anything.
+GP_ERR_INVALID_ARG before enqueueing anything, and so do GEMM calls of 8e10
+FLOP or more, whose shape decides whether they need it.
 """
 import pytest
 import torch
@@ -149,6 +150,46 @@ def test_linear_stage_graph_replays_match_eager(cuda):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), want.view(torch.int16)), f"replay {r}"
+
+
+@pytest.mark.parametrize("M,N,K", [(509, 512, 1024), (3000, 384, 192), (20000, 512, 512)])
+def test_gemm_graph_replays_match_eager(cuda, M, N, K):
+    """GEMM calls below 8e10 FLOP, on each of the tile sizes, allocate nothing."""
+    x = normal_fp16(M, K, seed=1, device=cuda)
+    w = (normal_fp16(K, N, seed=2, device=cuda).float() / K ** 0.5).half()
+    b = normal_fp16(1, N, seed=3, device=cuda)[0]
+    out = torch.empty((M, N), dtype=torch.float16, device=cuda)
+    gpipes.gemm_out(x, w, b, act="relu", out=out)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        gpipes.gemm_out(x, w, b, act="relu", out=out)
+    for r in range(3):
+        x.copy_(normal_fp16(M, K, seed=70 + r, device=cuda))
+        want = gpipes.gemm_out(x, w, b, act="relu")
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)), f"replay {r}"
+
+
+def test_large_gemm_refuses_capture_by_its_work(cuda):
+    """From 8e10 FLOP on: refused for the work, and the error says so (the call
+    takes no queue epoch)."""
+    M, N, K = 16384, 2048, 1280
+    x = normal_fp16(M, K, seed=1, device=cuda)
+    w = normal_fp16(K, N, seed=2, device=cuda)
+    out = gpipes.gemm_out(x, w)
+    torch.cuda.synchronize()
+    g, err = torch.cuda.CUDAGraph(), None
+    with torch.cuda.graph(g):
+        try:
+            gpipes.gemm_out(x, w, out=out)
+        except gpipes.GpipesError as e:
+            err = e
+    assert err is not None and err.code == -1 and "8e10 FLOP" in str(err) and "queue" not in str(err)
+    again = gpipes.gemm_out(x, w)
+    assert torch.equal(out.view(torch.int16), again.view(torch.int16))
 
 
 def test_nerf_noalloc_graph_replays_match_eager(cuda):
