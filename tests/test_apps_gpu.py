@@ -235,9 +235,11 @@ def test_nerf_a_rejects(cuda):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("act", ["none", "relu", "gelu_tanh", "sigmoid"])
 def test_ffn_fused_matches_chain(cuda, act, dtype):
-    """The one-kernel FFN blocks (H 128, FF 512) against the same block as GEMM and
-    LayerNorm calls: the pre-LayerNorm rows are the same 16-bit values, so outputs
-    agree but for the summation order of the statistics -- every element to one
+    """The one-kernel FFN blocks (H 128, FF 512) against the chain of GEMM launches
+    with the LayerNorm in their epilogues, which every other FF runs: padded to FF
+    640 with zero columns of w1, zeros of b1 and zero rows of w2 the block is the
+    same function, and the same bits.  Against the block as GEMM and LayerNorm
+    calls, whose statistics are summed in another order, every element to one
     rounding step (plus 2^-18 where the affine cancels), 99% of them bit for bit.
     Row counts around the 32-row tile and two tiles per CU; biases and affines
     present and absent; in place."""
@@ -249,6 +251,7 @@ def test_ffn_fused_matches_chain(cuda, act, dtype):
 
     w0, w1, w2 = rnd(H, H, k=H ** -0.5), rnd(H, FF, k=H ** -0.5), rnd(FF, H, k=FF ** -0.5)
     full = [rnd(H), rnd(FF), rnd(H), 1 + rnd(H, k=0.2), rnd(H, k=0.2), 1 + rnd(H, k=0.2), rnd(H, k=0.2)]
+    w1p, w2p = torch.cat([w1, w1.new_zeros(H, 128)], 1), torch.cat([w2, w2.new_zeros(128, H)])
     step = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
 
     def norm(v, ga, be):  # two-pass fp32 LayerNorm of 16-bit rows
@@ -267,8 +270,13 @@ def test_ffn_fused_matches_chain(cuda, act, dtype):
         ffn = lambda v: norm(gpipes.gemm_out(gpipes.gemm_out(v, w1, b1, act=act), w2, b2, r=v), ga2, be2)  # noqa: E731
         y = gpipes.bert_ffn(x, w1, b1, w2, b2, ga2, be2, act=act)
         close(y, ffn(x))
+        b1p = None if b1 is None else torch.cat([b1, b1.new_zeros(128)])
+        chain = gpipes.bert_ffn(x, w1p, b1p, w2p, b2, ga2, be2, act=act)
+        assert torch.equal(chain.view(torch.int16), y.view(torch.int16)), M
         # the second block from its own first LayerNorm's rows
         z = gpipes.bert_addln_ffn(attn, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, act=act)
+        chain = gpipes.bert_addln_ffn(attn, x, w0, b0, w1p, b1p, w2p, b2, ga0, be0, ga2, be2, act=act)
+        assert torch.equal(chain.view(torch.int16), z.view(torch.int16)), M
         h0 = norm(gpipes.gemm_out(attn, w0, b0, r=x), ga0, be0)
         want = ffn(h0)
         rows = torch.nonzero((z - want).abs().amax(1) > 0.1)  # a flipped rounding of h0 moves its row a little

@@ -95,15 +95,33 @@ def test_bert_ffn_no_affine_no_bias(cuda):
 
 
 # ------------------------------------------------------------------ LayerNorm in GEMM2's epilogue
-@pytest.mark.parametrize("M,H,FF", [(300, 128, 512), (257, 256, 1024), (1000, 512, 2048), (20000, 1024, 4096),
+def exchanges_statistics(call):
+    """Whether some launch of a bert_ffn call waits for another workgroup's LayerNorm
+    statistics: with every wait bounded to one poll such a call reports a timeout,
+    one whose LayerNorm is a launch of its own has no wait to fail."""
+    gpipes.set_wait_limit(1)
+    try:
+        call()
+        gpipes.pipeline_check()
+    except gpipes.GpipesError as e:
+        assert e.code == -5
+        return True
+    finally:
+        gpipes.set_wait_limit(0)
+    return False
+
+
+@pytest.mark.parametrize("M,H,FF", [(300, 128, 512), (300, 128, 384), (70000, 128, 384), (257, 256, 1024),
+                                    (1000, 512, 2048), (20000, 1024, 4096), (12000, 1024, 1024), (40000, 256, 512),
                                     (70000, 1024, 128), (100000, 512, 256)])
 def test_bert_ffn_ln_epilogue_matches_separate_launches(cuda, M, H, FF):
     """gp_bert_ffn_out computes the LayerNorm in GEMM2's epilogue: within a wave
-    at H = 128, from per-wave partial statistics exchanged between waves and
-    workgroups above (M = 20,000 at H = 1024 is two row chunks, two launches of
-    one exchange epoch; M = 70,000 at H = 1024, FF = 128 runs a 65,536-row chunk
-    as four rounds of 256 tiles in one launch, then a partial round; M = 100,000
-    at H = 512 four rounds, the last one partial).  Against GEMM2 + residual written out and the
+    at H = 128 (FF = 384; FF = 512 is one kernel for the block), from per-wave
+    partial statistics exchanged between waves and workgroups above (M = 20,000 at
+    H = 1024 is two row chunks, two launches of one exchange epoch; M = 70,000 at
+    H = 1024, FF = 128 runs a 65,536-row chunk as four rounds of 256 tiles in one
+    launch, then a partial round; M = 100,000 at H = 512 four rounds, the last one
+    partial) -- but for few rows (257 and 1000 here) in a launch of its own.  Against GEMM2 + residual written out and the
     LayerNorm launch reading it back, the pre-LayerNorm rows are the same fp16
     values and only the summation order of the statistics differs, so every
     output agrees to one fp16 rounding step and almost all bit for bit.  The
@@ -118,7 +136,9 @@ def test_bert_ffn_ln_epilogue_matches_separate_launches(cuda, M, H, FF):
     h = gpipes.gemm_out(x, p["w1"], p["b1"], act="gelu_tanh")
     pre = gpipes.gemm_out(h, p["w2"], p["b2"], r=x)
     sep = gpipes.layer_norm_out(pre, p["gamma"], p["beta"], eps=1e-12)
-    gpipes.pipeline_check()
+    if H > 128:
+        gpipes.pipeline_check()
+        assert exchanges_statistics(lambda: ffn(x, p, "gelu_tanh", 1e-12)) == (M > 1000)
     yf, sf = y.float(), sep.float()
     step = torch.maximum(yf.abs(), sf.abs()) * 2.0 ** -10 + 2.0 ** -18
     assert bool(((yf - sf).abs() <= step).all()), float((yf - sf).abs().max())
@@ -135,33 +155,59 @@ def test_bert_ffn_ln_exchange_reused_across_shapes(cuda):
     statistics, then calls with more row blocks and another width must still
     find their counters clean (a regression test: with the statistics placed
     right after the launch's own counters, the second call's counters held the
-    first call's statistics and its waits ran out)."""
+    first call's statistics and its waits ran out).  Calls of few rows, which take
+    no exchange area, run between them."""
     H, FF = 1024, 1024
     p = dev(bert_params(H, FF, seed=11, init="bert", affine_random=True), cuda)
     p2 = dev(bert_params(256, 512, seed=12, init="bert", affine_random=True), cuda)
-    for M, q, width in [(77, p, H), (1000, p, H), (3000, p2, 256), (600, p, H), (1000, p, H)]:
+    exchange = {(12000, H), (16384, H), (40000, 256)}
+    for M, q, width in [(12000, p, H), (77, p, H), (16384, p, H), (40000, p2, 256), (3000, p2, 256), (12000, p, H),
+                        (600, p, H), (16384, p, H)]:
         print(f"[ln-exchange] M={M} H={width}", flush=True)
         x = normal_fp16(M, width, seed=M, device=cuda)
         y = ffn(x, q, "gelu_tanh", 1e-12)
         gpipes.pipeline_check()
         rows = np.r_[0:min(M, 40), max(0, M - 40):M]
         assert_parity(f(y)[rows], oracle_ffn(x[rows], q, "gelu_tanh", 1e-12), f"reused exchange M={M} H={width}")
+    for M, q, width in ((12000, p, H), (16384, p, H), (40000, p2, 256), (77, p, H), (3000, p2, 256)):
+        x = normal_fp16(M, width, seed=M, device=cuda)
+        assert exchanges_statistics(lambda: ffn(x, q, "gelu_tanh", 1e-12)) == ((M, width) in exchange), M
 
 
-def test_bert_ffn_h128_tile_heights_agree(cuda):
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("FF", [384, 512, 640])
+def test_bert_ffn_h128_tile_heights_agree(cuda, FF, dtype):
     """At H = 128 a launch with fewer than 256 rows per CU runs its GEMM2 +
     LayerNorm on 128-row tiles, a larger one on 256-row tiles: the same
     products in the same order per row, so the rows of a small call equal the
-    same rows of a large one bit for bit (both against the oracle too)."""
+    same rows of a large one bit for bit (both against the oracle too).  FF = 512
+    is one kernel for the block at any row count; the block with the output
+    projection runs both of its LayerNorms on those tiles."""
     M = 80000
-    p = dev(bert_params(128, 512, seed=13, init="torch", affine_random=True), cuda)
-    x = normal_fp16(M, 128, seed=14, device=cuda)
-    big = ffn(x, p, "relu", 1e-5)
-    for r0, n in ((0, 300), (40000, 5000), (M - 1000, 1000)):
-        small = ffn(x[r0:r0 + n].contiguous(), p, "relu", 1e-5)
-        assert torch.equal(small.view(torch.int16), big[r0:r0 + n].view(torch.int16)), (r0, n)
+    p = {k: v.to(dtype) for k, v in dev(bert_params(128, FF, seed=13, init="torch", affine_random=True), cuda).items()}
+    x = normal_fp16(M, 128, seed=14, device=cuda, dtype=dtype)
+    attn = normal_fp16(M, 128, seed=15, device=cuda, dtype=dtype)
+    w0 = (normal_fp16(128, 128, seed=16, device=cuda).float() / 128 ** 0.5).to(dtype)
+
+    def addln(s):
+        return gpipes.bert_addln_ffn(attn[s], x[s], w0, p["b2"], p["w1"], p["b1"], p["w2"], p["b2"], p["gamma"],
+                                     p["beta"], p["gamma"], p["beta"], eps=1e-5, act="relu")
+
+    for call in (lambda s: ffn(x[s], p, "relu", 1e-5), addln):
+        big = call(slice(0, M))
+        for r0, n in ((0, 300), (40000, 5000), (M - 1000, 1000)):
+            small = call(slice(r0, r0 + n))
+            assert torch.equal(small.view(torch.int16), big[r0:r0 + n].view(torch.int16)), (r0, n)
     rows = np.r_[0:100, 40000:40100, M - 100:M]
-    assert_parity(f(big)[rows], oracle_ffn(x[rows], p, "relu", 1e-5), "H 128, 256-row tiles")
+    tol = (oracle.MAX_ABS_TOL, oracle.REL_L2_TOL) if dtype == torch.float16 else (oracle.BF16_MAX_ABS_TOL,
+                                                                                 oracle.BF16_REL_L2_TOL)
+    wants = (oracle_ffn(x[rows], p, "relu", 1e-5),
+             oracle.bert_addln_ffn(f(attn[rows]), f(x[rows]), f(w0), f(p["b2"]), f(p["w1"]), f(p["b1"]), f(p["w2"]),
+                                   f(p["b2"]), f(p["gamma"]), f(p["beta"]), f(p["gamma"]), f(p["beta"]),
+                                   act=oracle.ACT_RELU, eps=1e-5))
+    for got, want in zip((ffn(x, p, "relu", 1e-5), big), wants):
+        max_abs, rel = oracle.errors(f(got)[rows], want)
+        assert max_abs <= tol[0] and rel <= tol[1], (max_abs, rel)
 
 
 # ------------------------------------------------------------------ full size (config 2)
@@ -212,13 +258,11 @@ def test_gemm_residual(cuda, M, N, K):
     assert_parity(f(y0), oracle.linear(f(x), f(w), None) + f(r), f"gemm+residual no bias M={M}")
 
 
-def test_gemm_weight_paths_agree(cuda):
-    """Below 8e10 FLOP per call the GEMM reads the weights in their own [K, N]
-    layout (transposing LDS reads); above, it reads a transposed copy.  The
-    two compute the same products in the same order: a call above the limit
-    and the same rows in calls below it are bit-identical, and both match the
-    oracle on sampled rows."""
-    M, N, K = 16384, 2048, 1280  # 2 M N K = 8.6e10: the transposed copy
+def test_gemm_large_call_matches_its_parts(cuda):
+    """A call of 8.6e10 FLOP (256-row tiles) and the same rows in eight calls (128
+    x 128 tiles): the same products in the same order, so the same bits; sampled
+    rows against the oracle."""
+    M, N, K = 16384, 2048, 1280
     g = torch.Generator().manual_seed(17)
     x = torch.randn((M, K), generator=g).to(torch.float16).to(cuda)
     w = (torch.randn((K, N), generator=g) / np.sqrt(K)).to(torch.float16).to(cuda)
@@ -229,7 +273,37 @@ def test_gemm_weight_paths_agree(cuda):
     rows = np.r_[0:32, 8000:8032, M - 32:M]
     xs = f(x[torch.from_numpy(rows).to(cuda)])
     assert_parity(f(y[torch.from_numpy(rows).to(cuda)]), oracle.linear(xs, f(w), f(b), ACT_ID["gelu_tanh"]),
-                  "gemm transposed-copy path, sampled rows")
+                  "gemm large call, sampled rows")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N", [384, 512])
+@pytest.mark.parametrize("act", ["relu", "gelu_tanh"])
+def test_gemm_weight_paths_agree(cuda, N, act, dtype):
+    """The GEMM reads 16-byte aligned weights in their own [K, N] layout
+    (transposing LDS reads), others from a transposed copy.  The two compute the
+    same products in the same order: one MLP layer with its weight, or only its
+    bias, one element off alignment has the bits of the aligned call, at row counts
+    that run on each tile size (64, 128 and 256 rows), widths of whole and of half
+    256-feature tiles, K a whole number of slabs and not."""
+    for K in (320, 328, 64):
+        x = normal_fp16(40001, K, seed=K, device=cuda, dtype=dtype)
+        w = (normal_fp16(K, N, seed=N, device=cuda).float() / K ** 0.5).to(dtype)
+        b = normal_fp16(1, N, seed=5, device=cuda, dtype=dtype)[0]
+
+        def off(t):
+            u = torch.empty(t.numel() + 1, dtype=dtype, device=cuda)[1:].view(t.shape)
+            return u.copy_(t)
+
+        wu, bu = off(w), off(b)
+        assert wu.data_ptr() % 16 and bu.data_ptr() % 16
+        for M in (1, 65, 1500, 9001, 40001):
+            y = gpipes.mlp_out(x[:M], [w], [b], [act])
+            for ws, bs in (([wu], [b]), ([w], [bu]), ([wu], [bu])):
+                z = gpipes.mlp_out(x[:M], ws, bs, [act])
+                assert torch.equal(z.view(torch.int16), y.view(torch.int16)), (K, M)
+            if K % 64 == 0:
+                assert torch.equal(gpipes.gemm_out(x[:M], w, b, act=act).view(torch.int16), y.view(torch.int16)), (K, M)
 
 
 @pytest.mark.parametrize("M,N,K,act", [
