@@ -752,7 +752,12 @@ static hipError_t launch(const Args& a, int num_cus, hipStream_t s) {
 
 template <class C, bool BROW, typename E>
 static hipError_t dispatch(const Args& g, int act, int ncu, hipStream_t s) {
-  if (g.r) return act == ACT_NONE ? launch<C, ACT_NONE, true, BROW, 0, E>(g, ncu, s) : hipErrorInvalidValue;
+  // (No caller adds a residual behind a transposed copy of a 256-wide tile's weights.)
+  constexpr bool kResid = BROW || std::is_same_v<C, Narrow>;
+  if constexpr (kResid) {
+    if (g.r) return act == ACT_NONE ? launch<C, ACT_NONE, true, BROW, 0, E>(g, ncu, s) : hipErrorInvalidValue;
+  }
+  if (g.r) return hipErrorInvalidValue;
   switch (act) {
     case ACT_NONE: return launch<C, ACT_NONE, false, BROW, 0, E>(g, ncu, s);
     case ACT_RELU: return launch<C, ACT_RELU, false, BROW, 0, E>(g, ncu, s);
@@ -873,7 +878,7 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t s) {
       g.ln_target = (uint32_t)((a.ln_round + 1) * tiles_n * NW);
     }
   }
-  if (!a.ln)
+  if (!a.ln && (brow || !a.r))
     if (const int size = tile_cost(a.M, a.N, a.K, num_cus).size) return tile_launch(g, a.act, size, a.dtype, s);
   return a.dtype == GP_DTYPE_BF16 ? launch_typed<BF16>(a, g, brow, num_cus, s) : launch_typed<F16>(a, g, brow, num_cus, s);
 }

@@ -47,7 +47,8 @@ struct Args {
 };
 
 // Small-tile kernels (gemm_tile.hip): one `size` x `size` output tile per
-// workgroup (64 or 128); p.bt or p.w as in gemm_launch, no LayerNorm epilogue.
+// workgroup (64 or 128); p.bt or p.w as in gemm_launch (a residual with p.w
+// only), no LayerNorm epilogue.
 hipError_t tile_launch(const Args& p, int act, int size, int dtype, hipStream_t s);
 
 // Byte offset of logical 16-byte chunk c of unit row r: the chunk position is

@@ -342,24 +342,21 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(const half_t* x, const hal
       q = __builtin_fmaf(d, d, q);
     }
   q = pair_sum(q);
-  float m2 = q;
-  if constexpr (P > 1) {
-    float mp[P], qp[P];
+  float mp[P], qp[P];
 #pragma unroll
-    for (int i = 0; i < P; ++i) {
-      mp[i] = __shfl(mean, 2 * i, LPR);
-      qp[i] = __shfl(q, 2 * i, LPR);
-    }
-    mean = 0.f;
+  for (int i = 0; i < P; ++i) {
+    mp[i] = __shfl(mean, 2 * i, LPR);
+    qp[i] = __shfl(q, 2 * i, LPR);
+  }
+  mean = 0.f;
 #pragma unroll
-    for (int i = 0; i < P; ++i) mean += mp[i];
-    mean /= (float)P;
-    m2 = 0.f;
+  for (int i = 0; i < P; ++i) mean += mp[i];
+  mean /= (float)P;
+  float m2 = 0.f;
 #pragma unroll
-    for (int i = 0; i < P; ++i) {
-      const float d = mp[i] - mean;
-      m2 += __builtin_fmaf(128.f * d, d, qp[i]);
-    }
+  for (int i = 0; i < P; ++i) {
+    const float d = mp[i] - mean;
+    m2 += __builtin_fmaf(128.f * d, d, qp[i]);
   }
   const float rstd = rsqrtf(m2 / (float)N + eps);
   half_t* const orow = out + row * N + 128 * g;
@@ -397,7 +394,10 @@ static hipError_t launch(const Args& a, hipStream_t s) {
 
 template <class C, bool BROW, typename E>
 static hipError_t dispatch(const Args& g, int act, hipStream_t s) {
-  if (g.r) return act == ACT_NONE ? launch<C, ACT_NONE, true, BROW, E>(g, s) : hipErrorInvalidValue;
+  if constexpr (BROW) {
+    if (g.r) return act == ACT_NONE ? launch<C, ACT_NONE, true, BROW, E>(g, s) : hipErrorInvalidValue;
+  }
+  if (g.r) return hipErrorInvalidValue;
   switch (act) {
     case ACT_NONE: return launch<C, ACT_NONE, false, BROW, E>(g, s);
     case ACT_RELU: return launch<C, ACT_RELU, false, BROW, E>(g, s);
@@ -419,7 +419,6 @@ static hipError_t ln_typed(int64_t M, int64_t N, const half_t* x, const half_t* 
   const int64_t rows = 4 * kWave / (N / 64);  // rows per block
   const dim3 grid((unsigned)((M + rows - 1) / rows)), block(256);
   switch (N) {
-    case 128: hipLaunchKernelGGL((ln_rows_kernel<128, E>), grid, block, 0, s, x, g, b, eps, out, M); break;
     case 256: hipLaunchKernelGGL((ln_rows_kernel<256, E>), grid, block, 0, s, x, g, b, eps, out, M); break;
     case 512: hipLaunchKernelGGL((ln_rows_kernel<512, E>), grid, block, 0, s, x, g, b, eps, out, M); break;
     case 1024: hipLaunchKernelGGL((ln_rows_kernel<1024, E>), grid, block, 0, s, x, g, b, eps, out, M); break;

@@ -130,7 +130,7 @@ struct GemmArgs {
   const void* x;   // [M, lda]
   const void* wt;  // [N, K]
   const void* b;   // [N] or nullptr
-  const void* r;   // [M, ldr] residual or nullptr (then act must be ACT_NONE)
+  const void* r;   // [M, ldr] residual (act ACT_NONE; W in its own layout, or N an odd multiple of 128) or nullptr
   int act;
   void* out;       // [M, ldc]
   int64_t lda = 0, ldc = 0, ldr = 0;
@@ -174,7 +174,7 @@ size_t gemm_ln_ws_bytes(int64_t M, int64_t N);
 // LayerNorm in its epilogue: few rows, which the epilogue's 256-row tiles
 // would spread over few CUs.  The two give the same bits.
 bool gemm_ln_apart(int64_t M, int64_t N, int64_t K, int num_cus);
-// out = LayerNorm(x) over rows of N (128, 256, 512 or 1024) finished 16-bit
+// out = LayerNorm(x) over rows of N (256, 512 or 1024) finished 16-bit
 // values, with the statistics of the GEMM's LayerNorm epilogue bit for bit;
 // gamma / beta may be null (1 / 0).  In place when out == x.
 hipError_t gemm_ln_rows_launch(int64_t M, int64_t N, const void* x, const void* gamma, const void* beta, float eps,

@@ -150,9 +150,19 @@ int run_chain(int64_t M, int nl, const int64_t* widths, const void* const* w, co
   const int tl = nl - 2;  // first layer of the fused tail
   const bool fused_tail =
       widths[nl] == 1 && nl >= 2 && widths[nl - 1] == 256 && dlrm_tail_supported(widths[tl], acts[tl], acts[nl - 1]);
+  // Layers whose weights cannot be read in place, or not as fast, are transposed
+  // and padded into the workspace (one launch for all of them); the fused tail
+  // packs its own.
   Carve cv;
+  const int ngemm = fused_tail ? tl : nl;
+  std::vector<Prepared> L(nl);
   std::vector<size_t> o_wt(nl), o_b(nl);
-  for (int i = 0; i < nl; ++i) {
+  for (int i = 0; i < ngemm; ++i) {
+    if (in_place(widths[i + 1], w[i], b[i]) && !gemm_copy_weights(M, CH, np[i], kin[i], false, ncu)) {
+      L[i] = {nullptr, b[i], kin[i], np[i], acts[i], w[i], widths[i]};
+      continue;
+    }
+    L[i] = {nullptr, nullptr, kin[i], np[i], acts[i]};
     o_wt[i] = cv.take((size_t)np[i] * kin[i] * 2);
     o_b[i] = cv.take((size_t)np[i] * 2);
   }
@@ -163,19 +173,13 @@ int run_chain(int64_t M, int nl, const int64_t* widths, const void* const* w, co
   char* ws = nullptr;
   if ((rc = workspace_acquire(dev, s, cv.off, (void**)&ws))) return rc;
 
-  // Layers whose weights cannot be read in place are transposed and padded
-  // into the workspace (one launch for all of them); the fused tail packs its
-  // own.
-  std::vector<Prepared> L(nl);
   std::vector<PrepSpec> ps;
-  for (int i = 0; i < (fused_tail ? tl : nl); ++i) {
-    if (in_place(widths[i + 1], w[i], b[i]) && !gemm_copy_weights(M, CH, np[i], kin[i], false, ncu)) {
-      L[i] = {nullptr, b[i], kin[i], np[i], acts[i], w[i], widths[i]};
-    } else {
+  for (int i = 0; i < ngemm; ++i)
+    if (!L[i].w) {
       ps.push_back({w[i], ws + o_wt[i], b[i], ws + o_b[i], widths[i], widths[i + 1], kin[i], np[i]});
-      L[i] = {ws + o_wt[i], ws + o_b[i], kin[i], np[i], acts[i]};
+      L[i].wt = ws + o_wt[i];
+      L[i].b = ws + o_b[i];
     }
-  }
   if (!ps.empty())
     if (hipError_t e = prep_launch(ps.data(), (int)ps.size(), s); e != hipSuccess)
       return fail_hip(e, "MLP weight preparation");
