@@ -345,6 +345,22 @@ struct PhaseTimer {
 __device__ __forceinline__ unsigned long long phase_entry() { return 0; }
 #endif
 
+// Zeros for rows 16 n .. 16 n + 15 of every tile of an aborted workgroup, by the
+// stage-B wave that stores them, behind the stores it did issue (one that skipped
+// a store saw the abort word, which stays set).  Reads its coordinates anew, so
+// that nothing is kept in registers through the tile loop for it.
+__device__ __forceinline__ void zero_rows(const Params& p, int n) {
+  wait_vmcnt<0>();
+  const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+  const int64_t step = (int64_t)gridDim.x * TM;
+  for (int64_t row = (int64_t)blockIdx.x * TM + 16 * n + (lane >> 2); row - (lane >> 2) < p.M; row += step)
+    if (row < p.M) {
+      u32x4* const o = (u32x4*)(p.out + row * D + 32 * (lane & 3));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = u32x4{0, 0, 0, 0};
+    }
+}
+
 // GATHER_IDX: 0 = X given; 4 / 8 = gather, index bytes.  E: ElemF16 / ElemBF16.
 template <int K, bool LN, int GATHER_IDX = 0, typename E = ElemF16>
 __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -706,22 +722,14 @@ void mgn_fused_kernel(Params p) {
       tile_b((GP_LDS char*)hand0, k);
       if (k + 1 < nt) tile_b((GP_LDS char*)hand1, k + 1);
     }
-    // A wave that skipped a store saw the abort word, which stays set: it zeroes
-    // its sixteen rows of every tile, behind the stores it did issue.
-    if (p.fresh_out && lds_load_relaxed(ab) != 0) {
-      wait_vmcnt<0>();
-      for (int k = 0; k < nt; ++k) {
-        const int64_t grow = (t0 + (int64_t)k * G) * TM + 16 * n + l16;
-        const h4 zero[2] = {};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) store_row_pair(p.out + grow * D, zero, j, q4, grow < M);
-      }
-    }
     pt.finish(wave, lane, nt, t_entry, pro_t);
   }
   // The abort word is sticky and is set before the wave that set it gets
   // here, so the workgroup's timeout is reported at least once.
-  if (lds_load_relaxed(ab) != 0 && lane == 0) status_fail(p.status, p.epoch, kErrTimeout);
+  if (lds_load_relaxed(ab) != 0) {
+    if (lane == 0) status_fail(p.status, p.epoch, kErrTimeout);
+    if (p.fresh_out && !stage_a) zero_rows(p, n);
+  }
 }
 
 }  // namespace fused

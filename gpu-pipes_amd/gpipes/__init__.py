@@ -218,7 +218,7 @@ _FRESH = 0x100  # GP_OUT_FRESH
 
 def _new(x, impl, cols=None):
     """Output of an allocating form with x's rows: `cols` wide, or as wide as x."""
-    fused = _IMPLS.get(impl, impl) == IMPL_FUSED
+    fused = impl == "fused" or impl == IMPL_FUSED
     if cols is None:
         return torch.empty_like(x) if fused else torch.zeros_like(x)
     return (torch.empty if fused else torch.zeros)((x.shape[0], cols), dtype=x.dtype, device=x.device)
@@ -257,9 +257,12 @@ def _mgn_mlp(x, w1, b1, w2, b2, w3, b3, gamma, beta, out, eps, impl, fresh):
     with _on(x):
         args = (M, K, _ptr(x), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(w3), _ptr(b3), _ptr(gamma),
                 _ptr(beta), float(eps), _ptr(out), int(impl_id))
-        if impl_id != IMPL_FUSED:
-            fresh = 0
-        rc = lib.gp_mgn_mlp_dtype_out(*args, _DTYPES[dt] | fresh, _stream(x))
+        if fresh and impl_id == IMPL_FUSED:
+            rc = lib.gp_mgn_mlp_dtype_out(*args, _DTYPES[dt] | fresh, _stream(x))
+        elif dt == torch.float16:
+            rc = lib.gp_mgn_mlp_out(*args, _stream(x))
+        else:
+            rc = lib.gp_mgn_mlp_dtype_out(*args, _DTYPES[dt], _stream(x))
     _check(rc)
     return out
 
