@@ -595,8 +595,8 @@ def bench_chain(args):
                             "LN0, GEMM1 + act, GEMM2 + b2 + h0, LN2; pipelined: one queue-chained kernel)",
               "nerf_a": "one step: one gp_nerf_a_out call (fused: the weight-packing kernel, then the NeRF kernel "
                         "stopped after layer 8; pipelined: one queue-chained kernel)",
-              "bert_app": "one step: one gp_bert_ffn_impl_out call (fused: GEMM1 + b1 + act, GEMM2 + b2 + x with "
-                          "the LayerNorm in its epilogue; pipelined: one queue-chained kernel)"}
+              "bert_app": "one step: one gp_bert_ffn_impl_out call (fused: the weight-packing kernel, then one kernel "
+                          "of GEMM1 + b1 + act, GEMM2 + b2 + x and the LayerNorm; pipelined: one queue-chained kernel)"}
 
     call_ms, ms_per_step, settle = timed_steps(step, args, dev)
     avg_ms = sum(call_ms) / len(call_ms)

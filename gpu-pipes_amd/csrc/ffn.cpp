@@ -5,12 +5,13 @@
 // The reference's pipelined BERT FFN (apps/bert_ffn/pipelined/bert_ffn_pl.cuh:
 // 79-162) chains GEMM + bias + ReLU -> GEMM + bias with the residual as
 // accumulator -> LayerNorm workers through queues, sized for H = 128 and
-// FF = 512.  At BERT-large width the two GEMMs are compute-bound and their
-// weights cannot be held on chip, so here the block is three launches per row
-// chunk: GEMM1 with a bias + activation epilogue, GEMM2 with a bias +
-// residual epilogue, and the LayerNorm stage -- the shape of the reference's
-// bulk-sync variant (apps/bert_ffn/bulksync/bert_ffn_bs.cuh:12-27) with the add
-// fused.  Rows are processed in chunks so the FF-wide activations of one chunk
+// FF = 512; at that width either block is one kernel here (ffn_fused.hip).  At
+// BERT-large width the two GEMMs are compute-bound and their weights cannot be
+// held on chip, so the block is two launches per row chunk: GEMM1 with a bias +
+// activation epilogue and GEMM2 with a bias + residual + LayerNorm epilogue (for
+// few rows GEMM2 on small tiles and the LayerNorm behind it, gemm_ln_apart) --
+// the shape of the reference's bulk-sync variant
+// (apps/bert_ffn/bulksync/bert_ffn_bs.cuh:12-27) with the add fused.  Rows are processed in chunks so the FF-wide activations of one chunk
 // (at most 128 MiB: 16384 x 4096 at BERT-large width) can stay in the 256 MB
 // Infinity Cache between the two GEMMs rather than make a round trip through
 // HBM.

@@ -36,7 +36,13 @@
 // sits on one SIMD.  With the weights left in registers (wrong results) 16,384
 // rows take 13.5 instead of 15.2 us, so the feed is not it.  Kernel time of
 // bert_addln_ffn (fp16, ReLU): 100 rows 8.2 us, 16,384 rows 13.9, 32,768 rows
-// 21.6, against 40 us for the three GEMM launches at 32,768 rows.  Tried and
+// 21.6.  It is the faster way at large row counts too; us a call with the packing
+// launch, this kernel / the chain of GEMM launches (fp16):
+//   rows         FFN ReLU       FFN GELU       add + LN + FFN, ReLU / GELU
+//      32,768    19.9 / 31.3    21.1 / 31.8    24.1 / 41.1    26.5 / 42.0
+//     131,072    60.6 / 90.7    70.2 / 95.8    78.3 /  174    90.0 /  183
+//     300,000     131 /  245                    174 /  320
+//   1,048,576     460 /  763     581 /  831     601 / 1147     737 / 1241  Tried and
 // slower at 32,768 rows: three workgroups a CU with half the weights in flight
 // (23.4), eight waves on 64 rows (24.8).
 #include <hip/hip_runtime.h>

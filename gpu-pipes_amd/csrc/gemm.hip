@@ -786,8 +786,12 @@ static hipError_t launch_typed(const GemmArgs& a, Args& g, bool brow, int num_cu
 // per round of tiles over the CUs a K walk (microseconds per 64-k slab, more
 // when every CU copies at once) and an epilogue.  Fitted to 23 shapes, M 64 ..
 // 65,536, N 128 .. 4096, K 128 .. 4096 (fp16, weights in place, one kernel at
-// a time); within 15% of nearly all and with the fastest kernel of the three
-// on every one of them, e.g. 256-row / 128 x 128 / 64 x 64 tiles:
+// a time).  Over 473 other shapes, M 64 .. 262,143, N 128 .. 4096, K 64 .. 8192,
+// the kernel it picks is within 5% of the fastest of the three on 429 and within
+// 10% on 456.  The worst: N = 1024, K 192 .. 384 at 20,011 and 50,001 rows, where
+// 128 x 128 tiles would be 14 to 24% faster, and N = 384 at 50,001 rows (9 to 15%);
+// the kernel it picks there is the one that every call took before there was a
+// choice.  E.g. 256-row / 128 x 128 / 64 x 64 tiles:
 //   509 x 1024 x 4096    83 / 33 / 16 us     2048 x 1024 x 1024   27 / 12 / 10
 //   4096 x 1024 x 4096   87 / 39 / 65        8192 x 1024 x 4096   93 / 73 / 139
 //   4096 x 4096 x 1024   38 / 48 / 84        16384 x 1024 x 1024  37 / 41 / 56
@@ -807,7 +811,9 @@ static TileCost tile_cost(int64_t M, int64_t N, int64_t K, int num_cus) {
   // one ends do not wait for whole rounds.  256-row / 128 x 128 tiles, per call:
   // 50,001 x 128 -> 512 GELU 25.2 / 23.8 us, 100,000 x 128 -> 512 40.8 / 35.4,
   // 50,001 x 256 -> 1024 54.8 / 48.2.  At K = 256 and two rounds the two tie
-  // (50,001 x 256 -> 512 27.1 / 28.4, GELU 31.1 / 30.9).
+  // (50,001 x 256 -> 512 27.1 / 28.4, GELU 31.1 / 30.9).  Past K = 256 it goes
+  // either way with the fill of the last round (320 -> 512 at 50,001 rows 29.8 /
+  // 31.0 and at 100,003 60.7 / 57.0; 320 -> 1024 59.3 / 52.1 and 108 / 117).
   const bool shallow = wide && (K <= 128 || (K <= 256 && rounds(t256, 1) > 2)) && t256 > num_cus;
   const double c256 =
       5.0 + rounds(t256, 1) * (slabs * (wide ? 1.0 : 0.55) * (1.15 + 0.75 * load(t256)) + (shallow ? 5.3 : 3.0));

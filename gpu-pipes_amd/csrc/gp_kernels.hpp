@@ -80,7 +80,7 @@ struct BertFfnArgs {
 };
 
 // Either FFN block at the apps' width (H = 128, FF = 512) as one kernel
-// (ffn_fused.hip), any row count: the add + LayerNorm + FFN block, or with w0
+// (ffn_fused.hip; ahead of the GEMM chain from one row to a million): the add + LayerNorm + FFN block, or with w0
 // null the FFN block (attn = x; ga2 / be2 its affine).  All pointers 16-byte
 // aligned; the workspace (ffn_fused_workspace() bytes) receives the packed
 // weights.

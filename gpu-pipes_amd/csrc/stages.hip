@@ -299,8 +299,12 @@ static hipError_t launch_linear(const LinearArgs& a, int num_cus, hipStream_t s)
   constexpr int lds = gemm_stage_lds<MBLK, K, kLinearBufs>() + kGemmParamLds;
   // Workgroups per CU: at K = 128 LDS holds two, and one's weight prologue,
   // epilogue and last partial round run under the other's tiles (50,001 rows
-  // 9.1 -> 8.4 us, with LayerNorm 12.2 -> 10.6; 262,144 rows 29 -> 27.6 and 36 ->
-  // 31.5).  Wider inputs fill it alone.
+  // 9.1 -> 8.4 us, with LayerNorm 12.2 -> 10.6, kernel time; with an accumulator
+  // input 262,144 rows 44.5 -> 39.9 us a call, 1,048,576 rows 198 -> 160).  Without
+  // one, large calls differ between cards: at 262,144 rows one a CU
+  // takes 30 to 32 us everywhere, two take 29 to 36 (with LayerNorm 34 to 35 and 30
+  // to 40); a rule by rows that followed either kind lost on the other.  Wider
+  // inputs fill the LDS alone.
   constexpr int kPerCu = K == 128 ? 2 : 1;
   static_assert(kPerCu * lds <= 160 * 1024, "LDS");
   auto kern = linear_kernel<K, ACT, LN>;
