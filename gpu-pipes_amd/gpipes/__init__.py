@@ -771,10 +771,10 @@ def bert_addln_ffn_out(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, 
     """ln2(ffn(h0) + h0) with h0 = ln0(attn_out @ w0 + b0 + x), into ``out`` -- bert_addln_ffn_out of
     apps/bert_addln_ffn/pipelined/bert_addln_ffn_pl_ext.cu:17-58 (H 128, FF 512, ReLU, eps 1e-5
     there), for H in {128, 256, 512, 1024} and FF a multiple of 128.  Weights [in, out] =
-    ``weight.t().contiguous()``; biases and LayerNorm affines may be None.  impl "fused" (one
-    GEMM launch per layer with fused epilogues) or "pipelined" (the reference's queue-chained
-    layout, H 128 / FF 512 only).  Every tensor float16, or every tensor bfloat16 (fused impl
-    only: gp_bert_addln_ffn_dtype_out)."""
+    ``weight.t().contiguous()``; biases and LayerNorm affines may be None.  impl "fused" (at
+    H 128, FF 512 one kernel, else one GEMM launch per layer with fused epilogues) or
+    "pipelined" (the reference's queue-chained layout, H 128 / FF 512 only).  Every tensor
+    float16, or every tensor bfloat16 (fused impl only: gp_bert_addln_ffn_dtype_out)."""
     return _bert_addln_ffn(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0, ga2, be2, out, eps, act, impl, 0)
 
 

@@ -138,11 +138,13 @@ int gp_mgn_edge_gather_out(int64_t E, int64_t N, const void* nf, const void* ef,
  * Replaces bert_ffn_out(x, w1, b1, w2, b2, ga, be, out),
  * apps/bert_ffn/pipelined/bert_ffn_pl_ext.cu:24-56 (H = 128, FF = 512, ReLU,
  * eps 1e-5 fixed), and the bulk-sync chain gemm / gemm / add / LayerNorm of
- * apps/bert_ffn/bulksync/bert_ffn_bs.cuh:12-27.  Per row chunk, two GEMM
- * launches; the second computes the residual add and the LayerNorm in its
- * epilogue.  Above H = 128 a row spans several workgroups, which exchange
- * partial row statistics through the stream's queue arena with bounded waits:
- * such calls report failures through gp_pipeline_check.  Every workgroup of
+ * apps/bert_ffn/bulksync/bert_ffn_bs.cuh:12-27.  H = 128 with FF = 512 is one
+ * kernel; else, per row chunk, two GEMM launches, of which the second computes
+ * the residual add and the LayerNorm in its epilogue (calls of few rows: the
+ * LayerNorm in a launch of its own).  In the epilogue a row above H = 128 spans
+ * several workgroups, which exchange partial row statistics through the stream's
+ * queue arena with bounded waits: such calls report failures through
+ * gp_pipeline_check.  Every workgroup of
  * that launch (one per CU) must be resident at once, as for the queue-chained
  * layouts: kernels of other streams or processes holding CUs meanwhile can
  * make its waits run out (GP_ERR_TIMEOUT; never a hang).  The FF-wide
@@ -193,9 +195,9 @@ int gp_bert_ffn_dtype_out(int64_t M, int64_t H, int64_t FF, const void* x, const
  * Replaces bert_addln_ffn_out(attn_out, x, w0, b0, w1, b1, w2, b2, ga0, be0,
  * ga2, be2, out), apps/bert_addln_ffn/pipelined/bert_addln_ffn_pl_ext.cu:17-58
  * (H 128, FF 512, ReLU, M a multiple of 128).  impl GP_IMPL_FUSED (0, the
- * default) runs one GEMM launch per linear layer with bias, activation,
- * residual and LayerNorm fused into its epilogue, over row chunks in the
- * per-stream workspace (above H = 128 with failures reported by
+ * default) runs H = 128 with FF = 512 as one kernel, else one GEMM launch per
+ * linear layer with bias, activation, residual and LayerNorm fused into its
+ * epilogue, over row chunks in the per-stream workspace (above H = 128 with failures reported by
  * gp_pipeline_check, as gp_bert_ffn_out); GP_IMPL_PIPELINED runs the reference's
  * queue-chained layout (bert_addln_ffn_pl.cuh:92-176: stage workgroups linked
  * by ring queues, both adds fed from queues) for H = 128, FF = 512 and ReLU or
